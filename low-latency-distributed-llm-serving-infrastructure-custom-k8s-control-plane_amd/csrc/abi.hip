@@ -217,7 +217,7 @@ void paged_attention(const float* query, const float* key_cache, const float* va
   a.head_dim = dims.head_dim;
   a.scale_log2e = scaling * pa::kLog2e;
   g_ref_abi_status = from_hip(
-      pa::launch_generic(a, PA_DTYPE_F32, true, static_cast<hipStream_t>(stream)), "paged_attention");
+      pa::launch_flat(a, static_cast<hipStream_t>(stream)), "paged_attention");
 }
 
 size_t pa_pack_workspace_size(int32_t num_seqs) { return pa::pack_workspace_size(num_seqs); }
@@ -640,7 +640,7 @@ int decode_phases(const char* who, bool use_scratch, int32_t phases, const void*
   a.num_kv_heads = dims.num_kv_heads;
   a.head_dim = dims.head_dim;
   a.scale_log2e = scaling * pa::kLog2e;
-  return from_hip(pa::launch_generic(a, dims.dtype, false, s), who);
+  return from_hip(pa::launch_generic(a, dims.dtype, s), who);
 }
 
 }  // namespace
@@ -791,7 +791,7 @@ int prefill_impl(const char* who, const void* query, const void* key_cache, cons
   a.num_kv_heads = dims.num_kv_heads;
   a.head_dim = dims.head_dim;
   a.scale_log2e = scaling * pa::kLog2e;
-  return from_hip(pa::launch_generic(a, dims.dtype, false, s), who);
+  return from_hip(pa::launch_generic(a, dims.dtype, s), who);
 }
 
 }  // namespace

@@ -225,7 +225,10 @@ hipError_t launch_decode(const DecodeArgs& a, int dtype, int head_dim, int group
 hipError_t decode_workgroups_per_cu(int dtype, int head_dim, int group, bool pair, int* per_cu);
 
 bool generic_supported(int dtype, int head_dim);
-hipError_t launch_generic(const GenericArgs& a, int dtype, bool masked, hipStream_t stream);
+// Block-table source.
+hipError_t launch_generic(const GenericArgs& a, int dtype, hipStream_t stream);
+// fp32, gather/mask source (the reference ABI's call).
+hipError_t launch_flat(const GenericArgs& a, hipStream_t stream);
 
 size_t pack_workspace_size(int64_t num_seqs);
 // Whether one launch can pack the step: a single scan chunk, no gather or
