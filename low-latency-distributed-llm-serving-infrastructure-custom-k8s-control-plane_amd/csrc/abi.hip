@@ -397,20 +397,17 @@ int pa_swap_blocks(void* device_cache, void* host_cache, const int64_t* block_ma
 }
 
 namespace {
-// Two adjacent KV heads run as one workgroup reading one row of twice the
-// length per token (pa::decode_pairs_heads has the shapes).
-bool decode_pairs(const PaStepDims& d) {
-  const int group = d.num_kv_heads > 0 ? d.num_query_heads / d.num_kv_heads : 0;
-  return pa::decode_pairs_heads(d.dtype, d.head_dim, d.num_kv_heads, group);
+int unit_heads(const PaStepDims& d) {
+  return d.num_kv_heads > 0
+             ? pa::decode_unit_heads(d.dtype, d.head_dim, d.num_kv_heads, d.num_query_heads / d.num_kv_heads)
+             : 1;
 }
 // Bytes of merge records of a step: 8 per (sequence, decode unit,
 // sub-group), rounded up to 256 bytes.
 size_t merge_state_bytes(const PaStepDims& d) {
   if (d.num_seqs <= 0 || d.num_kv_heads <= 0 || d.num_query_heads < d.num_kv_heads) return 0;
   const int group = d.num_query_heads / d.num_kv_heads;
-  const bool pair = decode_pairs(d);
-  const int64_t units = (pair ? d.num_kv_heads / 2 : d.num_kv_heads) *
-                        static_cast<int64_t>(pair ? 1 : pa::decode_sub_groups(group));
+  const int64_t units = (d.num_kv_heads / unit_heads(d)) * static_cast<int64_t>(pa::decode_sub_groups(group));
   return (static_cast<size_t>(d.num_seqs) * units * 8 + 255) & ~size_t(255);
 }
 struct DecodeWorkspaceLayout {
@@ -442,9 +439,8 @@ int32_t pa_decode_workgroups_per_item(int32_t dtype, int32_t head_dim, int32_t n
                                       int32_t num_query_heads) {
   if (num_kv_heads <= 0 || num_query_heads <= 0 || num_query_heads % num_kv_heads != 0) return 0;
   const int group = num_query_heads / num_kv_heads;
-  if (pa::decode_pairs_heads(dtype, head_dim, num_kv_heads, group)) return num_kv_heads / 2;
   if (!pa::decode_fast_path_supported(dtype, head_dim, group, 16, 32)) return num_kv_heads;
-  return num_kv_heads * pa::decode_sub_groups(group);
+  return num_kv_heads / pa::decode_unit_heads(dtype, head_dim, num_kv_heads, group) * pa::decode_sub_groups(group);
 }
 
 int32_t pa_prefill_tile(int32_t num_query_heads, int32_t num_kv_heads) {
@@ -465,9 +461,8 @@ int32_t pa_decode_workgroups_per_cu(int32_t dtype, int32_t head_dim, int32_t num
          "head_dim %d, %d query heads per KV head", dtype, head_dim, group);
     return 0;
   }
-  const bool pair = pa::decode_pairs_heads(dtype, head_dim, num_kv_heads, group);
   int per_cu = 0;
-  const hipError_t err = pa::decode_workgroups_per_cu(dtype, head_dim, group, pair, &per_cu);
+  const hipError_t err = pa::decode_workgroups_per_cu(dtype, head_dim, num_kv_heads, group, &per_cu);
   if (err != hipSuccess) {
     from_hip(err, "pa_decode_workgroups_per_cu");
     return 0;
@@ -525,7 +520,6 @@ int decode_phases(const char* who, bool use_scratch, int32_t phases, const void*
   const int group = dims.num_query_heads / dims.num_kv_heads;
   const int eb = elem_bytes(dims.dtype);
   const int log2_bs = log2_exact(dims.block_size);
-  const bool pair = decode_pairs(dims);
   const bool fast =
       pa::decode_fast_path_supported(dims.dtype, dims.head_dim, group, dims.block_size,
                                      dims.partition_size) &&
@@ -589,14 +583,13 @@ int decode_phases(const char* who, bool use_scratch, int32_t phases, const void*
     a.merge_items = merge_items;
     a.num_merge = merge_items != nullptr ? num_merge_items : 0;
     a.block_table_stride = dims.max_blocks_per_seq;
-    a.num_kv_heads = pair ? dims.num_kv_heads / 2 : dims.num_kv_heads;
+    a.num_kv_heads = dims.num_kv_heads;
     a.total_blocks = dims.total_blocks;
     a.log2_block_size = log2_bs;
     a.partition = dims.partition_size;
     a.scale_log2e = scaling * pa::kLog2e;
-    a.pair = pair ? 1 : 0;
-    a.group = pair ? 2 * group : group;
-    a.sub_groups = pair ? 1 : pa::decode_sub_groups(group);
+    a.group = group;
+    a.sub_groups = pa::decode_workgroups_per_head(dims.dtype, dims.head_dim, group);
     a.head_dim = dims.head_dim;
     // A record's fields hold counts and items below 65535.
     a.merge_state = num_decode_items < 65535 ? merge_state : nullptr;

@@ -26,7 +26,7 @@ LIBRARY_NAME = "libpaged_attention_amd.so"
 LIBRARY_PATH = PACKAGE_DIR / LIBRARY_NAME
 OFFLOAD_ARCH = "gfx950"
 
-SOURCES = ["abi.hip", "plan.cpp", "pack.hip", "cache_write.hip", "decode.hip", "generic.hip", "prefill.hip",
+SOURCES = ["abi.hip", "plan.cpp", "pack.hip", "cache_write.hip", "decode.hip", "decode_mfma.hip", "generic.hip", "prefill.hip",
            "prefill256.hip", "prefill_f32.hip", "copy_blocks.hip", "calibrate.hip"]
 
 HIP_FLAGS = [

@@ -1,8 +1,10 @@
-// Paged-attention decode for gfx950: one workgroup per
+// Paged-attention decode for gfx950 on the vector units: one workgroup per
 // (sequence, context partition of up to 4096 tokens, KV head), split-K merge
-// after.  For bf16/fp16 with an even KV head count and up to 4 query heads per KV
-// head, two adjacent KV heads run as one workgroup that reads each token's
-// rows of both heads as one row of twice the length (see PAIR below).
+// after.  It serves fp32 caches, 16-bit heads of 80, 96 and 256, and 16-bit
+// heads of 64 and 128 in groups of up to 4 with an even KV head count: two
+// adjacent KV heads of those run as one workgroup that reads each token's
+// rows of both heads as one row of twice the length (see PAIR below).  The
+// other 16-bit heads of 64 and 128 run on the matrix cores (decode_mfma.hip).
 //
 // The workgroup (4 waves) serves the G = H_q / H_kv query heads that share
 // one KV head, so every K/V row of the partition is read from HBM once
@@ -42,16 +44,11 @@
 //
 // The reference computes the same quantity with its CPU loop nest
 // (csrc/src/paged_kernels.cpp:49-104) over a flat gather list and dense mask.
-#include "pa_common.hpp"
-#include "pa_launch.hpp"
+#include "decode_common.hpp"
 
 namespace pa {
 
-constexpr int kDecodeThreads = 256;
 constexpr int kMaxDecodeGroup = 8;  // query heads one unpaired workgroup serves
-constexpr int kDecodeWaves = kDecodeThreads / kWave;
-// Largest split-K partition (context tokens per workgroup) the kernel takes.
-constexpr int kMaxPartition = PA_DECODE_MAX_PARTITION;
 #ifndef PA_DECODE_TILE
 #define PA_DECODE_TILE 32  // context tokens per wave iteration (at least 2 rows per group)
 #endif
@@ -191,15 +188,6 @@ __device__ __forceinline__ float slice_dot(const uint4 (&q)[2], const uint4 (&k)
 }
 
 // Max over the lanes of a wave that share (lane % L): every row group.
-// gfx950 v_permlane16_swap / v_permlane32_swap with both operands = x:
-// element 0 holds rows {0,0,2,2} (halves {0,0}) and element 1 rows {1,1,3,3}
-// (halves {1,1}) of the 16-lane rows, so their max pairs rows (0,1),(2,3)
-// (resp. the two 32-lane halves).
-__device__ __forceinline__ float max_row_pairs(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
 // Every step pairs lanes of equal (lane % L) only (rotations by multiples of
 // L within a row of 16, then the row and half swaps), so the lanes of one
 // row group may hold different values (the reduce-scatter score layout).
@@ -211,81 +199,6 @@ __device__ __forceinline__ float across_groups_max(float x) {
   if constexpr (L <= 8) x = fmaxf(x, dpp<kDppRowRor8>(x));
   if constexpr (L <= 16) x = max_row_pairs(x);
   return max_halves(x);
-}
-
-// K output elements of one head of a multi-partition sequence from its
-// split-K partials: ml addresses the head's (max, sum) pair in item 0, acc
-// the first element's accumulator and out its output; element k sits
-// k * estride elements further.  Partitions 0 .. nfull-1 are items first ..
-// first + nfull - 1, partition nfull (when nparts > nfull) is item rem;
-// ml_stride / stride step one item.  kMergeBatch partitions per round trip,
-// with a running maximum (the stored maxima are already in the exp2
-// domain); slots past the last partition read the first one again and get
-// no weight.  The elements share each partial's (max, sum), loaded once for
-// all of them, and their loads go out together: one round trip per batch
-// for the K elements (one after the other, eight heads of 128 took four).
-// Each element's arithmetic is the same whatever K, and both merge paths
-// (the merge kernel, K = 1, and the in-launch merge of the partition
-// kernel) run this, so they give the same bits.
-constexpr int kMergeBatch = 8;
-constexpr int kMergeOutputs = 4;  // elements a thread of the in-launch merge merges at once
-
-// Partials read by the in-launch merge are written by workgroups on other
-// XCDs in the same launch: they are stored and loaded as device-scope
-// relaxed atomics, which write through and read past the XCD's L2, so no
-// L2 write-back or invalidate is needed (see the partition kernel's tail).
-__device__ __forceinline__ void store_device(float* p, float v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float load_device(const float* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-template <typename T, int K, bool DEVICE_LOADS = false>
-__device__ __forceinline__ void merge_partials(const float* ml, const float* acc, int estride, int64_t ml_stride,
-                                               int64_t stride, int64_t first, int nfull, int64_t rem, int nparts,
-                                               T* out) {
-  auto item_of = [&](int p) -> int64_t { return p < nfull ? first + p : rem; };
-  auto ld = [&](const float* q) { return DEVICE_LOADS ? load_device(q) : *q; };
-  float mx = kScoreFloor, sum = 0.f, o[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) o[k] = 0.f;
-  for (int p = 0; p < nparts; p += kMergeBatch) {
-    float mp[kMergeBatch], lp[kMergeBatch], xp[kMergeBatch][K];
-#pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u) {
-      const int64_t it = item_of(p + u < nparts ? p + u : 0);
-      mp[u] = ld(ml + it * ml_stride);
-      lp[u] = ld(ml + it * ml_stride + 1);
-#pragma unroll
-      for (int k = 0; k < K; ++k) xp[u][k] = ld(acc + it * stride + k * estride);
-    }
-    float mn = mx;
-#pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u) {
-      if (u > 0 && p + u >= nparts) {
-        mp[u] = kScoreFloor;
-        lp[u] = 0.f;
-#pragma unroll
-        for (int k = 0; k < K; ++k) xp[u][k] = 0.f;
-      }
-      mn = fmaxf(mn, mp[u]);
-    }
-    const float r = fast_exp2(mx - mn);
-    sum *= r;
-#pragma unroll
-    for (int k = 0; k < K; ++k) o[k] *= r;
-#pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u) {
-      const float w = fast_exp2(mp[u] - mn);
-      sum = fmaf(lp[u], w, sum);
-#pragma unroll
-      for (int k = 0; k < K; ++k) o[k] = fmaf(xp[u][k], w, o[k]);
-    }
-    mx = mn;
-  }
-#pragma unroll
-  for (int k = 0; k < K; ++k) store_scalar<T>(out + k * estride, sum > 0.f ? o[k] / sum : 0.f);
 }
 
 // PAIR: two adjacent real KV heads of D/2 run as one head of D with the G
@@ -1054,72 +967,15 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
   }
 
   // ---- in-launch split-K merge ---------------------------------------------
-  // The last of a sequence's partition workgroups (for this unit and
-  // sub-group) to finish merges the sequence's partials; no workgroup waits
-  // for another.  The workgroups run on different XCDs, whose L2s are
-  // separate: the partials above are device-scope stores (written through
-  // past the L2), and every wave waits for its stores to complete before
-  // the barrier.  Then one thread adds the workgroup's arrival to the
-  // sequence's 64-bit record with one device-scope atomic: bits 0-15 count
-  // arrivals, bits 16-39 hold 1 + the item of the partial last partition
-  // (added by that workgroup) and bits 40-63 1 + the item of partition 0,
-  // the first of the sequence's full partitions, which pa_pack lists as
-  // consecutive items (added by that workgroup; the host passes records
-  // only for fewer than 65535 items, so every field fits).  The workgroup
-  // whose addition brings the count to nparts has every field in the value
-  // the atomic returns; it resets the record for the next launch (the
-  // records start at zero and every launch leaves them at zero) and merges
-  // as the merge kernel does, with device-scope loads that read past its
-  // L2.  An agent-scope release or acquire fence here instead writes back or
-  // invalidates a whole L2 per workgroup, and made the decode slower than a
-  // second launch.
   if (nparts > 1 && n > 0 && a.merge_state != nullptr && seq >= 0 && seq < a.num_seqs) {
-    __shared__ int64_t s_merge[3];
-    const int nfull = ctx / a.partition;
-    const bool has_rem = nfull * a.partition < ctx;
-    uint64_t* rec = reinterpret_cast<uint64_t*>(a.merge_state) +
-                    ((static_cast<int64_t>(seq) * hkv + kvh) * a.sub_groups + sg);
-    uint64_t add = 1;
-    if (part == 0) add += static_cast<uint64_t>(item + 1) << 40;
-    if (part == nfull) add += static_cast<uint64_t>(item + 1) << 16;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (tid == 0) {
-      const uint64_t now = __hip_atomic_fetch_add(rec, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + add;
-      const bool last = static_cast<int>(now & 0xffff) == nparts;
-      if (last) {
-        __hip_atomic_store(rec, uint64_t{0}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_merge[1] = static_cast<int64_t>(now >> 40) - 1;
-        s_merge[2] = static_cast<int64_t>((now >> 16) & 0xffffff) - 1;
-      }
-      s_merge[0] = last;
-    }
-    __syncthreads();
-    if (s_merge[0]) {
-      const int64_t first = s_merge[1];
-      const int64_t rem = has_rem ? s_merge[2] : -1;
-      const bool ok = first >= 0 && first + nfull <= a.num_items && (!has_rem || (rem >= 0 && rem < a.num_items));
-      if (ok) {
-        // KC elements of one head per thread, ODM / KC apart, so that the
-        // lanes of a wave read consecutive floats of each partial; the
-        // thread's group r = tid, tid + 256, ... covers elements j + k *
-        // ODM / KC (k < KC) of head r / (ODM / KC), j = r % (ODM / KC).
-        // (fp32 heads of 80 and 96 take one at a time, which keeps their
-        // occupancy.)
-        constexpr int KO = (G * ODM + kDecodeThreads - 1) / kDecodeThreads;
-        constexpr int KM = MASKD && sizeof(T) == 4 ? 1 : kMergeOutputs;
-        constexpr int KC = KO >= 4 && KM >= 4 ? 4 : KO >= 2 && KM >= 2 ? 2 : 1;
-        constexpr int RUN = ODM / KC;  // groups per head
-        static_assert(ODM % KC == 0, "a group's elements stay inside one head");
-        for (int r = tid; r < G * RUN; r += kDecodeThreads) {
-          const int g = r / RUN;
-          const int e = g * ODM + (r - g * RUN);
-          merge_partials<T, KC, true>(a.part_ml + 2 * (h0 + g), a.part_acc + static_cast<int64_t>(h0) * ODM + e,
-                                      RUN, 2 * static_cast<int64_t>(hq), static_cast<int64_t>(hq) * ODM, first,
-                                      nfull, rem, nparts, out + e);
-        }
-      }
-    }
+    // (fp32 heads of 80 and 96 merge one element at a time, which keeps
+    // their occupancy.)
+    constexpr int KO = (G * ODM + kDecodeThreads - 1) / kDecodeThreads;
+    constexpr int KM = MASKD && sizeof(T) == 4 ? 1 : kMergeOutputs;
+    constexpr int KC = KO >= 4 && KM >= 4 ? 4 : KO >= 2 && KM >= 2 ? 2 : 1;
+    merge_in_launch<T, ODM, KC>(a, G, part, item, ctx, nparts,
+                                   (static_cast<int64_t>(seq) * hkv + kvh) * a.sub_groups + sg, h0, hq,
+                                   reinterpret_cast<T*>(a.output) + qtok * hq * ODM);
   }
 }
 
@@ -1157,6 +1013,26 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_merge_kernel(DecodeArgs
 
 // ---- host-side dispatch ------------------------------------------------
 
+// The merge phase, unless the partition launch merged in place (merge
+// records given): all a.group query heads of a KV head (or pair) merge in one
+// workgroup row; out_d: elements per query head in memory.
+template <typename T>
+static hipError_t launch_merge_t(const DecodeArgs& a, int out_d, int phases, hipStream_t stream) {
+  const int64_t grid = a.num_merge * a.num_kv_heads;
+  if (!(phases & PA_DECODE_PHASE_MERGE) || grid <= 0) return hipSuccess;
+  if ((phases & PA_DECODE_PHASE_PARTITIONS) && a.merge_state != nullptr) return hipSuccess;
+  const int chunks = (a.group * out_d + kDecodeThreads - 1) / kDecodeThreads;
+  hipLaunchKernelGGL((decode_merge_kernel<T>), dim3(static_cast<uint32_t>(grid), static_cast<uint32_t>(chunks)),
+                     dim3(kDecodeThreads), 0, stream, a, a.group, out_d);
+  return hipGetLastError();
+}
+
+static hipError_t launch_merge(const DecodeArgs& a, int dtype, int out_d, int phases, hipStream_t stream) {
+  return dtype == PA_DTYPE_BF16  ? launch_merge_t<bf16_t>(a, out_d, phases, stream)
+         : dtype == PA_DTYPE_F16 ? launch_merge_t<f16_t>(a, out_d, phases, stream)
+                                 : launch_merge_t<float>(a, out_d, phases, stream);
+}
+
 // Launches both phases of one kernel instance.  D, G: the kernel's head dim
 // and group (twice the real ones when paired).
 struct LaunchOp {
@@ -1167,24 +1043,14 @@ struct LaunchOp {
   template <typename T, int D, int G, bool PAIR, bool SHARED, int DM>
   hipError_t run() const {
     const int64_t grid = num_items * a.num_kv_heads * a.sub_groups;
-    const int64_t merge_grid = a.num_merge * a.num_kv_heads;
     if (phases & PA_DECODE_PHASE_PARTITIONS) {
       hipLaunchKernelGGL((decode_partition_kernel<T, D, G, PAIR, SHARED, DM>), dim3(static_cast<uint32_t>(grid)),
                          dim3(kDecodeThreads), 0, stream, a);
       const hipError_t err = hipGetLastError();
       if (err != hipSuccess) return err;
     }
-    if (!(phases & PA_DECODE_PHASE_MERGE) || merge_grid <= 0) return hipSuccess;
-    // The partition launch merged in place (merge records given).
-    if ((phases & PA_DECODE_PHASE_PARTITIONS) && a.merge_state != nullptr) return hipSuccess;
-    // Partials are in the real layout: rows of D/2 when paired; all a.group
-    // query heads of a KV head (or pair) merge in one workgroup row.
-    constexpr int kOutD = PAIR ? D / 2 : DM;
-    const int chunks = (a.group * kOutD + kDecodeThreads - 1) / kDecodeThreads;
-    hipLaunchKernelGGL((decode_merge_kernel<T>),
-                       dim3(static_cast<uint32_t>(merge_grid), static_cast<uint32_t>(chunks)),
-                       dim3(kDecodeThreads), 0, stream, a, a.group, kOutD);
-    return hipGetLastError();
+    // Partials are in the real layout: rows of D/2 when paired.
+    return launch_merge_t<T>(a, PAIR ? D / 2 : DM, phases, stream);
   }
 };
 
@@ -1225,14 +1091,10 @@ static hipError_t visit_group(int G, const Op& op) {
 template <bool SHARED, typename Op>
 static hipError_t visit_unpaired(int dtype, int head_dim, int g, const Op& op) {
   if (dtype == PA_DTYPE_BF16) {
-    if (head_dim == 128) return visit_group<bf16_t, 128, false, SHARED>(g, op);
-    if (head_dim == 64) return visit_group<bf16_t, 64, false, SHARED>(g, op);
     if (head_dim == 256) return visit_group<bf16_t, 256, false, SHARED>(g, op);
     if (head_dim == 96) return visit_group<bf16_t, 128, false, SHARED, 96>(g, op);
     if (head_dim == 80) return visit_group<bf16_t, 128, false, SHARED, 80>(g, op);
   } else if (dtype == PA_DTYPE_F16) {
-    if (head_dim == 128) return visit_group<f16_t, 128, false, SHARED>(g, op);
-    if (head_dim == 64) return visit_group<f16_t, 64, false, SHARED>(g, op);
     if (head_dim == 256) return visit_group<f16_t, 256, false, SHARED>(g, op);
     if (head_dim == 96) return visit_group<f16_t, 128, false, SHARED, 96>(g, op);
     if (head_dim == 80) return visit_group<f16_t, 128, false, SHARED, 80>(g, op);
@@ -1283,17 +1145,21 @@ static hipError_t visit_decode(int dtype, int head_dim, int group, bool pair, co
 #define PA_DECODE_PAIR_MAX_GROUP_D128 4
 #endif
 
-bool decode_pairs_heads(int dtype, int head_dim, int num_kv_heads, int group) {
-  if ((dtype != PA_DTYPE_BF16 && dtype != PA_DTYPE_F16) || num_kv_heads % 2 != 0 || group < 1)
-    return false;
-  if (head_dim == 64) return group <= PA_DECODE_PAIR_MAX_GROUP_D64;
-  if (head_dim == 128) return group <= PA_DECODE_PAIR_MAX_GROUP_D128;
-  return false;
+int decode_unit_heads(int dtype, int head_dim, int num_kv_heads, int group) {
+  if (!decode_uses_mfma(dtype, head_dim) || num_kv_heads % 2 != 0 || group < 1) return 1;
+  return group <= (head_dim == 64 ? PA_DECODE_PAIR_MAX_GROUP_D64 : PA_DECODE_PAIR_MAX_GROUP_D128) ? 2 : 1;
 }
 
 int decode_sub_groups(int group) {
   // The fewest equal sub-groups of at most kMaxDecodeGroup query heads.
   int n = (group + kMaxDecodeGroup - 1) / kMaxDecodeGroup;
+  while (n < group && group % n != 0) ++n;
+  return n > 0 ? n : 1;
+}
+
+int decode_workgroups_per_head(int dtype, int head_dim, int group) {
+  if (!decode_uses_mfma(dtype, head_dim)) return decode_sub_groups(group);
+  int n = (group + kMfmaHeads - 1) / kMfmaHeads;
   while (n < group && group % n != 0) ++n;
   return n > 0 ? n : 1;
 }
@@ -1314,11 +1180,31 @@ bool decode_fast_path_supported(int dtype, int head_dim, int group, int block_si
 hipError_t launch_decode(const DecodeArgs& a, int dtype, int head_dim, int group,
                          int64_t num_items, int phases, hipStream_t stream) {
   if (num_items <= 0) return hipSuccess;
-  return visit_decode(dtype, head_dim, group, a.pair != 0, LaunchOp{a, num_items, phases, stream});
+  if (decode_unit_heads(dtype, head_dim, a.num_kv_heads, group) == 2) {
+    DecodeArgs p = a;
+    p.num_kv_heads = a.num_kv_heads / 2;
+    p.group = 2 * a.group;
+    return visit_decode(dtype, head_dim, group, true, LaunchOp{p, num_items, phases, stream});
+  }
+  if (decode_uses_mfma(dtype, head_dim)) {
+    if (phases & PA_DECODE_PHASE_PARTITIONS) {
+      const hipError_t err = launch_decode_mfma(a, dtype, head_dim, num_items, stream);
+      if (err != hipSuccess) return err;
+    }
+    return launch_merge(a, dtype, head_dim, phases, stream);
+  }
+  return visit_decode(dtype, head_dim, group, false, LaunchOp{a, num_items, phases, stream});
 }
 
-hipError_t decode_workgroups_per_cu(int dtype, int head_dim, int group, bool pair, int* per_cu) {
+hipError_t decode_workgroups_per_cu(int dtype, int head_dim, int num_kv_heads, int group, int* per_cu) {
   *per_cu = 0;
+  const bool pair = decode_unit_heads(dtype, head_dim, num_kv_heads, group) == 2;
+  if (!pair && decode_uses_mfma(dtype, head_dim)) {
+    const int wgs = decode_workgroups_per_head(dtype, head_dim, group);
+    const hipError_t err = decode_mfma_workgroups_per_cu(dtype, head_dim, wgs > 1, per_cu);
+    *per_cu *= decode_sub_groups(group) / wgs;
+    return err;
+  }
   return visit_decode(dtype, head_dim, group, pair, OccupancyOp{per_cu});
 }
 

@@ -1,0 +1,477 @@
+// Paged-attention decode of 16-bit caches on the matrix cores: one workgroup
+// per (sequence, context partition, KV head), up to 16 query heads of the KV
+// head in one pass (larger groups run as sub-groups of at most 16).
+//
+// What bounds it is HBM: every K/V byte is read once for all 16 heads, and a
+// 32-token tile costs a wave 16 MFMAs and about 100 vector instructions
+// whatever the group.  The vector kernel (decode.hip) serves at most 8 heads a
+// pass (groups above 8 read K/V again through L2) at a dot2 per head, token
+// and pair of dims.  Vector kernel -> this one, steps of one layer: 48
+// sequences of 512-8192 tokens, 128/8 heads of 128, fp16, 227 -> 148 us (5.4
+// TB/s); 64 of 128-8192, 14/2 heads of 64, 39.3 -> 30.3 us; 256 of 32-8192,
+// 64/8 heads of 128, 734 -> 723 us (6.3 TB/s), 9/3 of 64, 144 -> 133 us.  A
+// workgroup alone reads three times as fast (8 sequences of 2048 tokens, 64/8
+// heads of 128 in whole partitions: 75 -> 25 us).
+//
+// v_mfma_f32_16x16x32: lane l = 16 c + r (c = 0..3) holds row r and the 8
+// k-values of its quarter c of the A operand, column r and the same k-values
+// of B, and column r, rows 4c .. 4c+3 of the result.  The order of k is free
+// as long as both operands agree, which makes the other operands a lane's
+// own registers:
+//  S^T = K Q^T   A: lane (r, c) holds token r's 16-byte pieces 4j + c, read
+//                from LDS, B: the same pieces of query head r (kept in
+//                registers).  The result gives the lane tokens 4c .. 4c+3 of
+//                head r.
+//  O^T = V^T P^T B: head r's probabilities of tokens 4c .. 4c+3 of both
+//                16-token halves of the tile -- the lane's own scores,
+//                exponentiated and packed, no exchange.  A: the same 8 tokens
+//                of V, which the lane loads as whole pieces (16 lanes read a
+//                row); dim PE * r + b of block b is then element b of the
+//                lane's pieces, so the transpose is v_perm_b32 on its own
+//                registers.  The result gives the lane PE * 4 consecutive
+//                dims of head r, whose softmax state it also holds.
+// K as operand loads straight from HBM (64 bytes of 16 rows an instruction,
+// no LDS) took 164 us in the first of those steps; streaming (nontemporal)
+// loads are worth 11-13 % where no sibling reads the rows again.
+// Each wave runs its own online softmax over every fourth tile, the next
+// tile's K and V loads in flight under the current tile's arithmetic, no
+// barrier in the loop.
+#include "decode_common.hpp"
+
+namespace pa {
+
+constexpr int kMfmaTile = 32;   // context tokens per wave iteration
+
+typedef float f32x4m __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8m __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8m __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4m __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2m __attribute__((ext_vector_type(2)));
+
+template <typename T>
+__device__ __forceinline__ f32x4m mfma16(u32x4m a, u32x4m b, f32x4m c);
+template <>
+__device__ __forceinline__ f32x4m mfma16<bf16_t>(u32x4m a, u32x4m b, f32x4m c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8m, a), __builtin_bit_cast(bf16x8m, b), c,
+                                                 0, 0, 0);
+}
+template <>
+__device__ __forceinline__ f32x4m mfma16<f16_t>(u32x4m a, u32x4m b, f32x4m c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8m, a), __builtin_bit_cast(f16x8m, b), c, 0,
+                                                0, 0);
+}
+
+// A lane's piece of a V row: D / 16 elements.
+template <int D>
+struct VPiece;
+template <>
+struct VPiece<64> {
+  using type = u32x2m;
+};
+template <>
+struct VPiece<128> {
+  using type = u32x4m;
+};
+
+// NT: streaming loads, for rows no other workgroup reads.
+template <typename V, bool NT>
+__device__ __forceinline__ V row_load(const void* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
+  return *reinterpret_cast<const V*>(p);
+}
+
+template <typename T, int D, bool SHARED>
+__global__ __launch_bounds__(kDecodeThreads) __attribute__((amdgpu_waves_per_eu(3))) void
+decode_mfma_kernel(DecodeArgs a) {
+  static_assert(sizeof(T) == 2, "16-bit caches");
+  constexpr bool kNt = !SHARED;
+  constexpr int KJ = D / 32;       // MFMAs of a 16-token half's scores
+  constexpr int PE = D / 16;       // V elements of a lane's piece, blocks of the output
+  constexpr int kRowBytes = D * 2;
+  constexpr int kAccRow = D + 4;   // padded LDS row of one head's accumulators
+  using VP = typename VPiece<D>::type;
+
+  __shared__ int s_blk[kMaxPartition + 2];
+  __shared__ float s_m[kDecodeWaves][kMfmaHeads];
+  __shared__ float s_l[kDecodeWaves][kMfmaHeads];
+  // Per wave: the K rows of its tile, and after the last tile its
+  // accumulators.
+  constexpr int kWaveBytes = kMfmaHeads * kAccRow * 4;
+  static_assert(kWaveBytes >= kMfmaTile * kRowBytes, "a tile's K rows fit");
+  __shared__ __align__(16) char s_wave[kDecodeWaves][kWaveBytes];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int r = lane & 15;  // token of a K load, query head elsewhere
+  const int c = lane >> 4;
+  const int hkv = a.num_kv_heads;
+  const int G = a.group / a.sub_groups;
+  // Workgroup -> (item, KV head, sub-group).  Ids are dealt to the XCDs
+  // round-robin: the members of a gang get ids that are equal modulo the XCD
+  // count and close together, gang after gang going to the next XCD (runs of
+  // 8 gangs, the last may be shorter).  Sub-groups that read the same rows
+  // form a gang, whose later reads hit that XCD's L2; so do all of an item's
+  // heads of 64, whose rows of 128 bytes share HBM bursts (128 sequences, 16/8
+  // heads: 208 -> 196 us), but not its heads of 128 (64 sequences, 32/32
+  // heads: 344 us spread over the XCDs, 357 as one gang).
+  const int gang_heads = D == 64 ? hkv : 1;
+  const int gang = gang_heads * a.sub_groups;
+  const int64_t run = blockIdx.x / (kXcds * gang);
+  const int at_run = static_cast<int>(blockIdx.x - run * (kXcds * gang));
+  const int width = static_cast<int>(min<int64_t>(kXcds, gridDim.x / gang - run * kXcds));
+  const int member = at_run / width;
+  const int64_t g_id = run * kXcds + (at_run - member * width);
+  const int64_t item = g_id / (hkv / gang_heads);
+  const int kvh = static_cast<int>(g_id - item * (hkv / gang_heads)) * gang_heads + member / a.sub_groups;
+  const int sg = member % a.sub_groups;
+  const int h0 = kvh * a.group + sg * G;  // first query head
+  const int seq = a.items[2 * item];
+  const int part = a.items[2 * item + 1];
+  const int64_t trow = a.rows != nullptr ? a.rows[seq] : seq;
+  const bool row_ok = trow >= 0 && trow < a.num_table_rows;
+  int ctx = a.context_lens[seq];
+  int64_t qtok = a.cu_seqlens[seq];
+  const int p0 = part * a.partition;
+  const int log2_bs = a.log2_block_size;
+  const int bs_mask = (1 << log2_bs) - 1;
+  // Block ids of the partition -> LDS (invalid ids become -1).  The whole
+  // span is read, whatever the context length, so that the reads do not wait
+  // for it.
+  const int first_blk = p0 >> log2_bs;
+  const int nblk = ((p0 + a.partition - 1) >> log2_bs) - first_blk + 1;
+  auto table_entry = [&](int i) {
+    const int col = first_blk + i;
+    return row_ok && col < a.block_table_stride ? a.block_tables[trow * a.block_table_stride + col] : -1;
+  };
+  auto valid_block = [&](int b) { return b < 0 || b >= a.total_blocks ? -1 : b; };
+  const int b0 = tid < nblk ? table_entry(tid) : -1;
+  // (both scalar loads issued before either is waited for: one round trip)
+  asm volatile("" : "+s"(ctx), "+s"(qtok));
+  const int n = max(0, min(a.partition, ctx - p0));
+  const int64_t row_bytes = static_cast<int64_t>(hkv) * kRowBytes;
+  const char* kbase = reinterpret_cast<const char*>(a.key_cache) + kvh * kRowBytes;
+  const char* vbase = reinterpret_cast<const char*>(a.value_cache) + kvh * kRowBytes;
+
+  // The query heads (zero past the group).
+  u32x4m q[KJ];
+#pragma unroll
+  for (int j = 0; j < KJ; ++j) {
+    const T* qrow = reinterpret_cast<const T*>(a.query) + qtok * a.q_token_stride +
+                    static_cast<int64_t>(h0 + min(r, G - 1)) * a.q_head_stride;
+    const u32x4m x = *reinterpret_cast<const u32x4m*>(qrow + (4 * j + c) * 8);
+    q[j] = r < G ? x : u32x4m{0, 0, 0, 0};
+  }
+
+  // pa_decode_append: the wave that attends the partition's last tile (which
+  // holds position ctx - 1) writes the new token's K and V rows of this KV
+  // head, a lane per 16-byte piece, just before that tile's loads; it loads
+  // the pieces here, beside the block ids.  No other wave or workgroup of the
+  // launch reads the position (sibling sub-groups write the same bytes).
+  constexpr int kAppendPieces = kRowBytes / 16;
+  const int ntiles = (n + kMfmaTile - 1) / kMfmaTile;
+  const bool append = a.new_key != nullptr && n > 0 && p0 + n == ctx;
+  const bool append_wave = append && (ntiles - 1) % kDecodeWaves == wave;
+  char* append_dst = nullptr;
+  uint4 append_piece = make_uint4(0, 0, 0, 0);
+  if (append_wave && lane < 2 * kAppendPieces) {
+    const int col = (ctx - 1) >> log2_bs;
+    const int b = row_ok && col < a.block_table_stride ? a.block_tables[trow * a.block_table_stride + col] : -1;
+    if (b >= 0 && b < a.total_blocks) {
+      const bool is_v = lane >= kAppendPieces;
+      const int e = (is_v ? lane - kAppendPieces : lane) * 8;
+      append_piece = ld16(reinterpret_cast<const T*>(is_v ? a.new_value : a.new_key) +
+                          qtok * (is_v ? a.new_value_token_stride : a.new_key_token_stride) +
+                          static_cast<int64_t>(kvh) * (is_v ? a.new_value_head_stride : a.new_key_head_stride) + e);
+      const int64_t slot = (static_cast<int64_t>(b) << log2_bs) + ((ctx - 1) & bs_mask);
+      append_dst = const_cast<char*>(is_v ? vbase : kbase) + slot * row_bytes + e * 2;
+    }
+  }
+
+  bool hole = false;  // a block the partition needs is missing
+  {
+    auto stage = [&](int i, int b) {
+      s_blk[i] = b;
+      hole |= b < 0 && (i << log2_bs) < n + (p0 & bs_mask);
+    };
+    if (tid < nblk) stage(tid, valid_block(b0));
+    for (int i = tid + kDecodeThreads; i < nblk; i += kDecodeThreads) stage(i, valid_block(table_entry(i)));
+  }
+  hole = __syncthreads_or(hole);
+
+  VP vt[8];  // V of a tile: tokens 4c .. 4c+3 of the first half, then of the second
+  // K goes straight into LDS, whole rows per load (in the operand's layout a
+  // load would touch 64 bytes of 16 rows, 12 % slower), the 16-byte chunks of
+  // token t at position chunk ^ swizzle(t), which spreads the 16 rows of an
+  // operand read over the banks.
+  constexpr int kChunks = kRowBytes / 16;
+  constexpr int kRowsPerLoad = kWave / kChunks;
+  constexpr int kLoads = 16 / kRowsPerLoad;  // per 16-token half
+  auto swizzle = [](int t) { return kChunks == 16 ? 4 * (t & 3) + ((t >> 2) & 3) : (t >> 1) & 7; };
+  char* const s_k = s_wave[wave];
+  // Row of the lane within load i of a half, and its bytes from the half's
+  // first row.
+  auto k_row = [&](int i) { return kRowsPerLoad * i + lane / kChunks; };
+  auto k_chunk = [&](int i) { return static_cast<uint32_t>(((lane % kChunks) ^ swizzle(k_row(i))) * 16); };
+  auto load_k_lds = [&](const char* src, int s, int i) {
+    typedef const __attribute__((address_space(1))) void* global_ptr;
+    typedef __attribute__((address_space(3))) void* lds_ptr;
+    __builtin_amdgcn_global_load_lds((global_ptr)(src), (lds_ptr)(s_k + (s * kLoads + i) * (kWave * 16)), 16, 0,
+                                     kNt ? 2 : 0);
+  };
+  uint32_t koff[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) koff[i] = static_cast<uint32_t>(k_row(i) * static_cast<int>(row_bytes)) + k_chunk(i);
+  const uint32_t voff = static_cast<uint32_t>(4 * c * static_cast<int>(row_bytes) + r * (PE * 2));
+  auto write_new_rows = [&](int tile) {
+    if (append_wave && tile == ntiles - 1) {
+      if (append_dst != nullptr) st16(append_dst, append_piece);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    }
+  };
+  // Blocks of 16 tokens or more, all of them there: a 16-token half lies in
+  // one block, so it takes one scalar base and per-lane offsets.  Tokens past
+  // the partition's end read rows of its last half's block.
+  int64_t at[2];  // byte offset of each half's first row
+  auto locate = [&](int tile) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int t = min(tile * kMfmaTile + 16 * s, (n - 1) & ~15);
+      const int b = __builtin_amdgcn_readfirstlane(s_blk[((p0 + t) >> log2_bs) - first_blk]);
+      at[s] = ((static_cast<int64_t>(b) << log2_bs) | ((p0 + t) & bs_mask)) * row_bytes;
+    }
+  };
+  auto load_k = [&]() {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) load_k_lds(kbase + at[s] + koff[i], s, i);
+  };
+  auto load_v = [&]() {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vt[4 * s + i] = row_load<VP, kNt>(vbase + at[s] + i * row_bytes + voff);
+  };
+  // Any block size, blocks missing: a slot per lane; a token without a block
+  // (or past the end) reads slot 0.
+  auto slot_of = [&](int t) -> int64_t {
+    const int b = t < n ? s_blk[((p0 + t) >> log2_bs) - first_blk] : -1;
+    return b < 0 ? 0 : (static_cast<int64_t>(b) << log2_bs) | ((p0 + t) & bs_mask);
+  };
+  auto load_any = [&](int tile) {
+    const int t0 = tile * kMfmaTile;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        load_k_lds(kbase + slot_of(t0 + 16 * s + k_row(i)) * row_bytes + k_chunk(i), s, i);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        vt[4 * s + i] = row_load<VP, kNt>(vbase + slot_of(t0 + 16 * s + 4 * c + i) * row_bytes + r * (PE * 2));
+    }
+  };
+
+  const float scale = a.scale_log2e;
+  float m = kScoreFloor, l = 0.f;  // head r; l: this lane's tokens only
+  f32x4m acc[PE];                  // acc[b][i]: dim PE * (4c + i) + b of head r
+#pragma unroll
+  for (int b = 0; b < PE; ++b) acc[b] = f32x4m{0.f, 0.f, 0.f, 0.f};
+
+  f32x4m s[2];  // scores of tokens 4c .. 4c+3 of each half, head r
+  auto scores = [&]() {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      s[h] = f32x4m{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < KJ; ++j) {
+        const int at_chunk = (4 * j + c) ^ swizzle(r);
+        s[h] = mfma16<T>(*reinterpret_cast<const u32x4m*>(s_k + (16 * h + r) * kRowBytes + 16 * at_chunk), q[j], s[h]);
+      }
+    }
+  };
+  // Tokens past the end or without a block get no weight, and their V rows
+  // (uninitialised or infinite, perhaps) are zeroed.
+  auto mask = [&](int tile) {
+    const int t = tile * kMfmaTile + (lane & (kMfmaTile - 1));
+    const uint32_t live =
+        static_cast<uint32_t>(__ballot(t < n && s_blk[((p0 + min(t, n - 1)) >> log2_bs) - first_blk] >= 0));
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool on = (live >> (16 * h + 4 * c + i)) & 1u;
+        s[h][i] = on ? s[h][i] : -INFINITY;
+        if (!on) vt[4 * h + i] = VP{};
+      }
+  };
+  auto attend = [&]() {
+    float tm = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
+                     fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
+    tm = max_halves(max_row_pairs(tm));
+    const float m_new = fmaxf(m, tm);
+    if (__any(m_new != m)) {
+      const float alpha = fast_exp2((m - m_new) * scale);
+      l *= alpha;
+#pragma unroll
+      for (int b = 0; b < PE; ++b) acc[b] *= alpha;
+      m = m_new;
+    }
+    const float mc = -m * scale;
+    u32x4m p;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float pa = fast_exp2(fmaf(s[h][2 * i], scale, mc));
+        const float pb = fast_exp2(fmaf(s[h][2 * i + 1], scale, mc));
+        l += pa + pb;
+        p[2 * h + i] = pack_half2<T>(pa, pb);
+      }
+#pragma unroll
+    for (int w = 0; w < PE / 2; ++w) {
+      u32x4m lo, hi;  // elements 2w and 2w + 1 of the 8 tokens
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        lo[i] = __builtin_amdgcn_perm(vt[2 * i + 1][w], vt[2 * i][w], 0x05040100u);
+        hi[i] = __builtin_amdgcn_perm(vt[2 * i + 1][w], vt[2 * i][w], 0x07060302u);
+      }
+      acc[2 * w] = mfma16<T>(lo, p, acc[2 * w]);
+      acc[2 * w + 1] = mfma16<T>(hi, p, acc[2 * w + 1]);
+    }
+  };
+
+  if (wave < ntiles) {
+    int tile = wave;
+    if (log2_bs < 4 || hole) {
+      for (; tile < ntiles; tile += kDecodeWaves) {
+        write_new_rows(tile);
+        load_any(tile);
+        scores();
+        mask(tile);
+        attend();
+      }
+    } else {
+      // The next tile's K loads go out once the scores have used the current
+      // K, its V loads once the product has used the current V: one register
+      // set, both always in flight.  (The scheduling barriers keep them there.)
+      write_new_rows(tile);
+      locate(tile);
+      load_k();
+      __builtin_amdgcn_sched_barrier(0);
+      load_v();
+      __builtin_amdgcn_sched_barrier(0);
+      for (; tile + kDecodeWaves < ntiles; tile += kDecodeWaves) {
+        locate(tile + kDecodeWaves);
+        scores();
+        write_new_rows(tile + kDecodeWaves);
+        __builtin_amdgcn_sched_barrier(0);
+        load_k();
+        __builtin_amdgcn_sched_barrier(0);
+        attend();
+        load_v();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      scores();
+      mask(tile);
+      attend();
+    }
+  }
+
+  // ---- combine the waves -------------------------------------------------
+  l = sum_halves(sum_row_pairs(l));
+  float* acc_row = reinterpret_cast<float*>(s_k) + r * kAccRow + 4 * PE * c;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int b = 0; b < PE; b += 4)
+      *reinterpret_cast<float4*>(acc_row + PE * i + b) =
+          make_float4(acc[b][i], acc[b + 1][i], acc[b + 2][i], acc[b + 3][i]);
+  if (lane < kMfmaHeads) {
+    s_m[wave][lane] = m * scale;
+    s_l[wave][lane] = l;
+  }
+  __syncthreads();
+
+  const int hq = hkv * a.group;
+  const int nparts = (ctx + a.partition - 1) / a.partition;
+  float* pacc = a.part_acc + (item * hq + h0) * D;
+  T* out = reinterpret_cast<T*>(a.output) + (qtok * hq + h0) * D;
+  for (int i = tid; i < G * D; i += kDecodeThreads) {
+    const int g = i / D;
+    const int e = g * kAccRow + (i - g * D);
+    float mx = s_m[0][g];
+#pragma unroll
+    for (int w = 1; w < kDecodeWaves; ++w) mx = fmaxf(mx, s_m[w][g]);
+    float o = 0.f, sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < kDecodeWaves; ++w) {
+      const float f = fast_exp2(s_m[w][g] - mx);
+      o = fmaf(reinterpret_cast<const float*>(s_wave[w])[e], f, o);
+      sum = fmaf(s_l[w][g], f, sum);
+    }
+    if (nparts <= 1) {
+      store_scalar<T>(out + i, sum > 0.f ? o / sum : 0.f);
+    } else {
+      store_device(pacc + i, o);
+      if (i % D == 0) {
+        float* pml = a.part_ml + (item * hq + h0 + g) * 2;
+        store_device(pml, mx);
+        store_device(pml + 1, sum);
+      }
+    }
+  }
+  if (nparts > 1 && n > 0 && a.merge_state != nullptr && seq >= 0 && seq < a.num_seqs)
+    merge_in_launch<T, D, kMergeOutputs>(a, G, part, item, ctx, nparts,
+                                         (static_cast<int64_t>(seq) * hkv + kvh) * a.sub_groups + sg, h0, hq,
+                                         reinterpret_cast<T*>(a.output) + qtok * hq * D);
+}
+
+bool decode_uses_mfma(int dtype, int head_dim) {
+  return (dtype == PA_DTYPE_BF16 || dtype == PA_DTYPE_F16) && (head_dim == 64 || head_dim == 128);
+}
+
+template <typename Op>
+static hipError_t visit_mfma(int dtype, int head_dim, bool shared, const Op& op) {
+  if (dtype == PA_DTYPE_BF16) {
+    if (head_dim == 128) return shared ? op.template run<bf16_t, 128, true>() : op.template run<bf16_t, 128, false>();
+    if (head_dim == 64) return shared ? op.template run<bf16_t, 64, true>() : op.template run<bf16_t, 64, false>();
+  } else if (dtype == PA_DTYPE_F16) {
+    if (head_dim == 128) return shared ? op.template run<f16_t, 128, true>() : op.template run<f16_t, 128, false>();
+    if (head_dim == 64) return shared ? op.template run<f16_t, 64, true>() : op.template run<f16_t, 64, false>();
+  }
+  return hipErrorNotSupported;
+}
+
+struct MfmaLaunch {
+  const DecodeArgs& a;
+  int64_t num_items;
+  hipStream_t stream;
+  template <typename T, int D, bool SHARED>
+  hipError_t run() const {
+    const int64_t grid = num_items * a.num_kv_heads * a.sub_groups;
+    hipLaunchKernelGGL((decode_mfma_kernel<T, D, SHARED>), dim3(static_cast<uint32_t>(grid)), dim3(kDecodeThreads), 0,
+                       stream, a);
+    return hipGetLastError();
+  }
+};
+
+struct MfmaOccupancy {
+  int* per_cu;
+  template <typename T, int D, bool SHARED>
+  hipError_t run() const {
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, decode_mfma_kernel<T, D, SHARED>, kDecodeThreads, 0);
+  }
+};
+
+hipError_t launch_decode_mfma(const DecodeArgs& a, int dtype, int head_dim, int64_t num_items, hipStream_t stream) {
+  return visit_mfma(dtype, head_dim, a.sub_groups > 1, MfmaLaunch{a, num_items, stream});
+}
+
+hipError_t decode_mfma_workgroups_per_cu(int dtype, int head_dim, bool shared, int* per_cu) {
+  return visit_mfma(dtype, head_dim, shared, MfmaOccupancy{per_cu});
+}
+
+}  // namespace pa

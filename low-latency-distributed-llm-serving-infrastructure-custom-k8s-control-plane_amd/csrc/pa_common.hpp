@@ -188,8 +188,13 @@ __device__ __forceinline__ float sum_halves(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Sum of rows (0,1) and (2,3) of the four 16-lane rows (v_permlane16_swap,
-// both operands = x), at every lane position.
+// Max / sum of rows (0,1) and (2,3) of the four 16-lane rows.  gfx950
+// v_permlane16_swap with both operands = x: element 0 holds rows {0,0,2,2}
+// and element 1 rows {1,1,3,3} at every lane position.
+__device__ __forceinline__ float max_row_pairs(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
 __device__ __forceinline__ float sum_row_pairs(float x) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);

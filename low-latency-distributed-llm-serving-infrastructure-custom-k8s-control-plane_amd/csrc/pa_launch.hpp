@@ -32,13 +32,9 @@ struct DecodeArgs {
   int32_t log2_block_size;
   int32_t partition;
   float scale_log2e;
-  // 1: two adjacent real KV heads of D/2 run as one of D (G counts the query
-  // heads of both).  Every query head reads only its own half of the rows;
-  // outputs and partials use the real layout [.., H_q, D/2].
-  int32_t pair;
-  // Query heads per num_kv_heads unit (for a pair, those of both heads) and
-  // the workgroups that share them (1 unless the group is split because it
-  // exceeds the largest kernel group; each then re-reads the unit's K/V).
+  // Query heads per KV head and the workgroups that share them (1 unless the
+  // group is split because it exceeds the largest kernel group; each then
+  // re-reads the head's K/V).
   int32_t group;
   int32_t sub_groups;
   // pa_decode_append: the step's new K/V rows ([T, H_kv, head_dim], element
@@ -51,7 +47,7 @@ struct DecodeArgs {
   int64_t new_key_head_stride;
   int64_t new_value_token_stride;
   int64_t new_value_head_stride;
-  int32_t head_dim;  // real head dim (the pair's unit row holds two heads)
+  int32_t head_dim;
   // Merge records of the in-launch split-K merge, 8 bytes per (sequence,
   // unit, sub-group): arrivals, first full-partition item, partial item.
   // Zero before the launch and left zero by it; null (always for 65535 or
@@ -213,16 +209,22 @@ constexpr int kMaxDecodeQueryGroup = 64;
 // Workgroups sharing one KV head's query heads: the fewest equal sub-groups
 // of at most 8 heads.
 int decode_sub_groups(int group);
-// Whether two adjacent KV heads of this shape run as one workgroup
-// (DecodeArgs::pair; the KV head count must then be even).
-bool decode_pairs_heads(int dtype, int head_dim, int num_kv_heads, int group);
-// phases: PA_DECODE_PHASE_PARTITIONS and/or PA_DECODE_PHASE_MERGE.  head_dim
-// and group are the real ones; a.num_kv_heads counts pairs when a.pair.
+// Workgroups one KV head's query heads take in the decode launch: the
+// sub-groups, or fewer where the matrix-core kernel serves up to 16 heads a
+// workgroup (the unit count stays that of the sub-groups).
+int decode_workgroups_per_head(int dtype, int head_dim, int group);
+// Adjacent KV heads that run as one workgroup: 2 for 16-bit heads of 64 and
+// 128 in groups of up to 4 with an even KV head count, else 1.  Such units are
+// what pa_decode_workgroups_per_item counts (times the sub-groups) and what
+// merge records are kept for.
+int decode_unit_heads(int dtype, int head_dim, int num_kv_heads, int group);
+// phases: PA_DECODE_PHASE_PARTITIONS and/or PA_DECODE_PHASE_MERGE;
+// head_dim and group are the model's.
 hipError_t launch_decode(const DecodeArgs& a, int dtype, int head_dim, int group,
                          int64_t num_items, int phases, hipStream_t stream);
-// Resident partition workgroups per CU of the kernel launch_decode runs for
-// a shape (the HIP occupancy calculator on the current device).
-hipError_t decode_workgroups_per_cu(int dtype, int head_dim, int group, bool pair, int* per_cu);
+// Resident units per CU of the kernel a launch that fills the chip runs (the HIP
+// occupancy calculator on the current device).
+hipError_t decode_workgroups_per_cu(int dtype, int head_dim, int num_kv_heads, int group, int* per_cu);
 
 bool generic_supported(int dtype, int head_dim);
 // Block-table source.
