@@ -1,10 +1,7 @@
 // Paged-attention decode for gfx950 on the vector units: one workgroup per
 // (sequence, context partition of up to 4096 tokens, KV head), split-K merge
-// after.  It serves fp32 caches, 16-bit heads of 80, 96 and 256, and 16-bit
-// heads of 64 and 128 in groups of up to 4 with an even KV head count: two
-// adjacent KV heads of those run as one workgroup that reads each token's
-// rows of both heads as one row of twice the length (see PAIR below).  The
-// other 16-bit heads of 64 and 128 run on the matrix cores (decode_mfma.hip).
+// after.  fp32 caches and 16-bit heads of 80, 96 and 256 run here; 16-bit
+// heads of 64 and 128 run on the matrix cores (decode_mfma.hip).
 //
 // The workgroup (4 waves) serves the G = H_q / H_kv query heads that share
 // one KV head, so every K/V row of the partition is read from HBM once
@@ -48,7 +45,7 @@
 
 namespace pa {
 
-constexpr int kMaxDecodeGroup = 8;  // query heads one unpaired workgroup serves
+constexpr int kMaxDecodeGroup = 8;  // query heads one workgroup serves
 #ifndef PA_DECODE_TILE
 #define PA_DECODE_TILE 32  // context tokens per wave iteration (at least 2 rows per group)
 #endif
@@ -68,17 +65,14 @@ constexpr int kMaxDecodeGroup = 8;  // query heads one unpaired workgroup serves
 #ifndef PA_DECODE_MIN_WAVES_WIDE
 #define PA_DECODE_MIN_WAVES_WIDE 2  // the same for wider groups or rows
 #endif
-#ifndef PA_DECODE_MIN_WAVES_PAIR512
-#define PA_DECODE_MIN_WAVES_PAIR512 3  // the same for 16-bit rows of 512 bytes (pairs, D 256)
+#ifndef PA_DECODE_MIN_WAVES_ROW512
+#define PA_DECODE_MIN_WAVES_ROW512 3  // the same for 16-bit rows of 512 bytes (D 256)
 #endif
-// GA: query heads whose accumulators one lane holds (G, or G/2 when paired,
-// whose rows of up to 512 bytes come in half-length tiles).
-#define PA_DECODE_OCCUPANCY(T, D, GA, PAIR)                                                  \
-  __attribute__((amdgpu_waves_per_eu(                                                        \
-      ((GA) <= 4 && ((PAIR) || sizeof(T) == 2) && (D) * sizeof(T) > 256)                     \
-          ? PA_DECODE_MIN_WAVES_PAIR512                                                      \
-      : ((GA) <= 4 && ((D) * sizeof(T) <= 256 || (PAIR))) ? PA_DECODE_MIN_WAVES              \
-                                                          : PA_DECODE_MIN_WAVES_WIDE)))
+#define PA_DECODE_OCCUPANCY(T, D, G)                                                          \
+  __attribute__((amdgpu_waves_per_eu(                                                         \
+      ((G) <= 4 && sizeof(T) == 2 && (D) * sizeof(T) > 256) ? PA_DECODE_MIN_WAVES_ROW512      \
+      : ((G) <= 4 && (D) * sizeof(T) <= 256)                ? PA_DECODE_MIN_WAVES             \
+                                                            : PA_DECODE_MIN_WAVES_WIDE)))
 
 typedef unsigned int u32x2v __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
@@ -148,17 +142,6 @@ struct VRaw<8> {
   using type = uint2;
 };
 
-// Dot product of one 16-byte piece of K with the matching piece of q
-// (16-bit elements).
-template <typename T>
-__device__ __forceinline__ float piece_dot(uint4 q, uint4 k) {
-  static_assert(Elem<T>::kBytes == 2, "paired heads have 16-bit elements");
-  float acc = dot2_half<T>(q.x, k.x, 0.f);
-  acc = dot2_half<T>(q.y, k.y, acc);
-  acc = dot2_half<T>(q.z, k.z, acc);
-  return dot2_half<T>(q.w, k.w, acc);
-}
-
 // 32-bit word w of a lane's V piece (a pair of 16-bit elements).
 __device__ __forceinline__ uint32_t v_word(uint32_t v, int) { return v; }
 __device__ __forceinline__ uint32_t v_word(uint2 v, int w) { return w == 0 ? v.x : v.y; }
@@ -201,18 +184,6 @@ __device__ __forceinline__ float across_groups_max(float x) {
   return max_halves(x);
 }
 
-// PAIR: two adjacent real KV heads of D/2 run as one head of D with the G
-// query heads of both (the first G/2 belong to the first real head); every
-// query head reads only its own real head's half of the rows.  QK layout:
-//  - rows of 512 bytes ("split"): the first half of a row group's lanes holds
-//    the first real head's half of the row (two pieces per lane, as for an
-//    unpaired row), the second half the other's; a lane scores the G/2 heads
-//    of its own real head, summed over L/2 lanes.
-//  - rows of 256 bytes: every lane's first piece lies in the first real
-//    head's half and its second piece in the other's (so each wave load still
-//    reads 128-byte runs); each head dots its own piece, summed over L lanes.
-// PV layout: lanes [0, 32) hold the first half of the row, and each lane
-// accumulates only the G/2 heads of its half.
 // SHARED: the workgroup is one of several sub-groups of a KV head's query
 // heads, whose siblings read the same K/V rows (cached loads).
 // DM: the head dim in memory, when smaller than the lane layout's D (heads
@@ -220,11 +191,10 @@ __device__ __forceinline__ float across_groups_max(float x) {
 // past DM read the row's first piece or slice instead (always in bounds);
 // their q pieces are zero, so those K pieces add nothing to the scores, and
 // their accumulators are never stored.
-template <typename T, int D, int G, bool PAIR, bool SHARED, int DM>
-__global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G / 2 : G), PAIR) void decode_partition_kernel(DecodeArgs a) {
+template <typename T, int D, int G, bool SHARED, int DM>
+__global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void decode_partition_kernel(DecodeArgs a) {
   // Tiles of 16 tokens for wide groups and for 16-bit rows of 512 bytes
-  // (pairs of heads of 128, heads of 256: the same bytes per tile as 32
-  // tokens of 256-byte rows).
+  // (the same bytes per tile as 32 tokens of 256-byte rows).
   using S = DecodeShape<T, D,
                         ((G > 4 || (Elem<T>::kBytes == 2 && D * sizeof(T) > 256)) ? PA_DECODE_TILE_WIDE
                                                                                    : PA_DECODE_TILE)>;
@@ -244,21 +214,16 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
   // p staging per wave: 16-bit pairs [16 pairs][G] or fp32 [32 tokens][G]
   constexpr int kTile = S::kTile;
   constexpr int PWORDS = HALF ? (kTile / 2) * G : kTile * G;
-  constexpr int GA = PAIR ? G / 2 : G;    // heads a lane accumulates
-  constexpr int OUT_D = PAIR ? D / 2 : D;  // s_acc elements per query head
   constexpr bool MASKD = DM < D;
-  constexpr int ODM = PAIR ? D / 2 : DM;  // output elements per query head in memory
   constexpr int KPM = DM / S::kChunkElems;  // 16-byte pieces of a row in memory
-  static_assert(!MASKD || (!PAIR && DM % S::kChunkElems == 0 && KPM >= S::kL && DM % S::kPe == 0),
-                "masked head dims: unpaired, whole 16-byte pieces, at least one piece per lane");
-  static_assert(!PAIR || (HALF && G % 2 == 0 && S::kR == 1 && S::kTpg >= 1),
-                "pairs: 16-bit elements, an even head count, one V row per wave load");
-  // RS: reduce-scatter scores, for unpaired groups of more than half a row
+  static_assert(!MASKD || (DM % S::kChunkElems == 0 && KPM >= S::kL && DM % S::kPe == 0),
+                "masked head dims: whole 16-byte pieces, at least one piece per lane");
+  // RS: reduce-scatter scores, for groups of more than half a row
   // group of lanes (L of 4 or 8): NP score positions (G rounded up to a power
   // of two, at least L), and lane lig of every row group ends with the
   // scores of its HPL query heads lig*HPL .. lig*HPL + HPL-1 alone (see
   // qk_softmax_rs).
-  constexpr bool RS = !PAIR && (L == 4 || L == 8) && G > L / 2;
+  constexpr bool RS = (L == 4 || L == 8) && G > L / 2;
   constexpr int NP = !RS ? 1 : (G <= L ? L : 8);
   constexpr int HPL = RS ? NP / L : 1;
 
@@ -272,7 +237,7 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
   __shared__ uint32_t s_p[kDecodeWaves][PWORDS];
   __shared__ float s_m[kDecodeWaves][G];
   __shared__ float s_l[kDecodeWaves][G];
-  __shared__ float s_acc[kDecodeWaves][G * OUT_D];
+  __shared__ float s_acc[kDecodeWaves][G * D];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -333,8 +298,8 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
   const T* vbase = reinterpret_cast<const T*>(a.value_cache) + kvh * DM;
 
   // pa_decode_append: the workgroups of the partition holding the new token
-  // (position ctx - 1) write its K and V rows of this unit (one KV head, or
-  // the pair's two) into the cache, as pa_reshape_and_cache would; sibling
+  // (position ctx - 1) write its K and V rows of this KV head into
+  // the cache, as pa_reshape_and_cache would; sibling
   // sub-groups write the same bytes.  The wave that attends the partition's
   // last tile (the one holding that position) does it, a lane per 16-byte
   // piece: it loads the piece here, so the load overlaps the staging below,
@@ -384,7 +349,6 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
   const int lig = lane % L;  // lane within its row group
   const int gi = lane / L;   // row group within the wave
   constexpr int QCHUNKS = G * D / CE;  // 16-byte pieces of the G query rows
-  constexpr int HC = D / CE / 2;  // 16-byte pieces of a real head when paired
   constexpr int QN = RS ? 2 * L * NP : QCHUNKS;  // 16-byte pieces staged
   auto query_piece = [&](int i) -> uint4 {
     if constexpr (RS) {
@@ -404,13 +368,7 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
       const int c = i - g * (D / CE);
       const T* qrow = reinterpret_cast<const T*>(a.query) + qtok * a.q_token_stride +
                       static_cast<int64_t>(h0 + g) * a.q_head_stride;
-      if constexpr (PAIR) {
-        // Query head g belongs to real KV head g / GA of the pair: its D/2
-        // elements go into that half of the row (the other half is never read).
-        return (c / HC) == (g / GA) ? ld16(qrow + (c % HC) * CE) : make_uint4(0, 0, 0, 0);
-      } else {
-        return (!MASKD || c < KPM) ? ld16(qrow + c * CE) : make_uint4(0, 0, 0, 0);
-      }
+      return (!MASKD || c < KPM) ? ld16(qrow + c * CE) : make_uint4(0, 0, 0, 0);
     }
   };
   // Each thread's first table entry and first query piece are both loaded
@@ -446,37 +404,25 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
   const float scale = a.scale_log2e;
   const int sub = lane / S::kLp;  // V row of this lane within a wave load
   const int lp = lane % S::kLp;   // head-dimension slice of this lane
-  // Paired: which real head's half of the row the lane's V slice lies in.
-  const int hh = PAIR ? lp / (S::kLp / 2) : 0;
-  float m[G], acc[GA][PE];
+  float m[G], acc[G][PE];
 #pragma unroll
   for (int g = 0; g < G; ++g) m[g] = kScoreFloor;
 #pragma unroll
-  for (int j = 0; j < GA; ++j)
+  for (int j = 0; j < G; ++j)
 #pragma unroll
     for (int e = 0; e < PE; ++e) acc[j][e] = 0.f;
 
   // ---- per-tile work ------------------------------------------------------
-  // A lane computes the scores of NS query heads, summed over LS lanes: all
-  // G over the row group, or, in the split pair layout, the G/2 of its own
-  // real head over its half of the group.  Its K pieces are kp0 and
-  // kp0 + KP1 (16-byte pieces of the row).
-  constexpr bool SPLIT = PAIR && D * sizeof(T) > 256;
-  constexpr int NS = SPLIT ? GA : G;
-  constexpr int LS = SPLIT ? L / 2 : L;
-  constexpr int KP1 = SPLIT ? L / 2 : L;
-  const int khalf = SPLIT ? lig / LS : 0;              // real head of the lane's pieces
-  const int kp0 = SPLIT ? khalf * L + lig % LS : lig;  // first 16-byte piece of the lane
-  const int gq0 = SPLIT ? khalf * GA : 0;              // first query head it scores
-  // Softmax exponentials are spread over the LS lanes that share those
-  // scores: lane lig owns "combos" k = lig % LS + LS*r, each one (token pair,
+  // A lane's K pieces are lig and lig + L (16-byte pieces of the row).
+  // Softmax exponentials are spread over the L lanes of a row group: lane
+  // lig owns "combos" k = lig + L*r, each one (token pair,
   // head) for bf16 or (token, head) for fp32, and computes, sums and stages
   // only those.
-  constexpr int NC = (HALF ? TPG / 2 : TPG) * NS;  // combos per lane group
-  constexpr int CPL = (NC + LS - 1) / LS;          // combos per lane
-  float lsum[NS];  // this lane's share of the softmax denominators of its NS heads
+  constexpr int NC = (HALF ? TPG / 2 : TPG) * G;  // combos per lane group
+  constexpr int CPL = (NC + L - 1) / L;           // combos per lane
+  float lsum[G];  // this lane's share of the softmax denominators
 #pragma unroll
-  for (int j = 0; j < NS; ++j) lsum[j] = 0.f;
+  for (int j = 0; j < G; ++j) lsum[j] = 0.f;
   float ml[HPL];  // RS: running maxima of the lane's own heads (sums in lsum[0 .. HPL-1])
 #pragma unroll
   for (int h = 0; h < HPL; ++h) ml[h] = kScoreFloor;
@@ -491,9 +437,9 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
   };
   // Per-lane element offset of its K slice within a wave load: row group gi
   // reads row gi of the load (GPW consecutive tokens).
-  const int64_t koff = static_cast<int64_t>(gi) * row_stride + kp0 * CE;
+  const int64_t koff = static_cast<int64_t>(gi) * row_stride + lig * CE;
   // Second K piece of the lane (its first piece again past DM).
-  const int kp1 = (!MASKD || kp0 + KP1 < KPM) ? kp0 + KP1 : kp0;
+  const int kp1 = (!MASKD || lig + L < KPM) ? lig + L : lig;
   const bool k_uniform = log2_bs >= S::kLog2Gpw;  // a load's GPW tokens share a block
   auto issue_k = [&](int tile, int blk_lane) {
     const int t0 = tile * kTile;
@@ -511,7 +457,7 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
               (static_cast<int64_t>(b) << log2_bs) | ((p0 + t0 + GPW * i) & bs_mask);
           const T* row = kbase + slot0 * row_stride + koff;
           kb[i][0] = kv_load<uint4, kNt>(row);
-          kb[i][1] = kv_load<uint4, kNt>(row + (MASKD ? (kp1 - kp0) * CE : KP1 * CE));
+          kb[i][1] = kv_load<uint4, kNt>(row + (MASKD ? (kp1 - lig) * CE : L * CE));
         } else {
           kb[i][0] = make_uint4(0, 0, 0, 0);
           kb[i][1] = make_uint4(0, 0, 0, 0);
@@ -523,8 +469,8 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
         if (kok[i]) {
           const int64_t slot = (static_cast<int64_t>(b) << log2_bs) | ((p0 + t) & bs_mask);
           const T* row = kbase + slot * row_stride;
-          kb[i][0] = kv_load<uint4, kNt>(row + kp0 * CE);
-          kb[i][1] = kv_load<uint4, kNt>(row + (MASKD ? kp1 : kp0 + KP1) * CE);
+          kb[i][0] = kv_load<uint4, kNt>(row + lig * CE);
+          kb[i][1] = kv_load<uint4, kNt>(row + (MASKD ? kp1 : lig + L) * CE);
         } else {
           kb[i][0] = make_uint4(0, 0, 0, 0);
           kb[i][1] = make_uint4(0, 0, 0, 0);
@@ -678,7 +624,7 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
 #pragma unroll
       for (int h = 0; h < HPL; ++h) lsum[h] *= fast_exp2((ml[h] - ml_new[h]) * scale);
 #pragma unroll
-      for (int j = 0; j < GA; ++j)
+      for (int j = 0; j < G; ++j)
 #pragma unroll
         for (int e = 0; e < PE; ++e) acc[j][e] *= alpha[j];
     }
@@ -711,46 +657,28 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
   };
 
   auto qk_softmax = [&](bool full) {
-    float s[TPG][NS];
-    float tmax[NS];
+    float s[TPG][G];
+    float tmax[G];
 #pragma unroll
-    for (int j = 0; j < NS; ++j) tmax[j] = -INFINITY;
+    for (int j = 0; j < G; ++j) tmax[j] = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < NS; ++j) {
-      uint4 qg[2];
-      if constexpr (PAIR && !SPLIT) {
-        // Head j's own piece: piece 0 for the first G/2 heads, piece 1 after.
-        qg[0] = s_q[j * (D / CE) + (j / GA) * L + lig];
-      } else {
-        qg[0] = s_q[(gq0 + j) * (D / CE) + kp0];
-        qg[1] = s_q[(gq0 + j) * (D / CE) + kp0 + KP1];
-      }
+    for (int j = 0; j < G; ++j) {
+      const uint4 qg[2] = {s_q[j * (D / CE) + lig], s_q[j * (D / CE) + lig + L]};
 #pragma unroll
       for (int i = 0; i < TPG; ++i) {
-        float v;
-        if constexpr (PAIR && !SPLIT) v = group_sum<L>(piece_dot<T>(qg[0], kb[i][j / GA]));
-        else v = group_sum<LS>(slice_dot<T>(qg, kb[i]));
+        float v = group_sum<L>(slice_dot<T>(qg, kb[i]));
         if (!full) v = kok[i] ? v : -INFINITY;
         s[i][j] = v;
         tmax[j] = fmaxf(tmax[j], v);
       }
     }
-    // Tile maxima over the row groups.  In the split pair layout head g's is
-    // held by lane 0, or, for the second real head, by lane LS (the first
-    // lane of the second half of row group 0).
+    // Tile maxima over the row groups.
     bool moved = false;
     float m_new[G];
-    float red[NS];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      if constexpr (SPLIT) {
-        if (g < GA) red[g] = across_groups_max<L>(tmax[g]);
-        m_new[g] = fmaxf(m[g], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(red[g % GA]),
-                                                                          g < GA ? 0 : LS)));
-      } else {
-        m_new[g] = __int_as_float(__builtin_amdgcn_readfirstlane(
-            __float_as_int(fmaxf(m[g], across_groups_max<L>(tmax[g])))));
-      }
+      m_new[g] = __int_as_float(
+          __builtin_amdgcn_readfirstlane(__float_as_int(fmaxf(m[g], across_groups_max<L>(tmax[g])))));
       moved |= m_new[g] != m[g];
     }
     if (moved) {  // wave-uniform
@@ -758,19 +686,13 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         alpha[g] = fast_exp2((m[g] - m_new[g]) * scale);
-        if constexpr (!SPLIT) lsum[g] *= alpha[g];
+        lsum[g] *= alpha[g];
         m[g] = m_new[g];
       }
-      if constexpr (SPLIT) {
 #pragma unroll
-        for (int j = 0; j < GA; ++j) lsum[j] *= khalf ? alpha[GA + j] : alpha[j];
-      }
+      for (int j = 0; j < G; ++j)
 #pragma unroll
-      for (int j = 0; j < GA; ++j) {
-        const float al = PAIR ? (hh ? alpha[GA + j] : alpha[j]) : alpha[j];
-#pragma unroll
-        for (int e = 0; e < PE; ++e) acc[j][e] *= al;
-      }
+        for (int e = 0; e < PE; ++e) acc[j][e] *= alpha[j];
     }
     float mneg[G];
 #pragma unroll
@@ -778,34 +700,33 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
     uint32_t* sp = s_p[wave];
 #pragma unroll
     for (int r = 0; r < CPL; ++r) {
-      const int c = (SPLIT ? lig % LS : lig) + LS * r;
-      if (NC % LS != 0 && c >= NC) break;
+      const int c = lig + L * r;
+      if (NC % L != 0 && c >= NC) break;
       float sa = -INFINITY, sb = -INFINITY, mc = 0.f;  // mc: -max * scale of the head
 #pragma unroll
       for (int cc = 0; cc < NC; ++cc) {
         const bool mine = c == cc;
         if constexpr (HALF) {
-          sa = mine ? s[2 * (cc / NS)][cc % NS] : sa;
-          sb = mine ? s[2 * (cc / NS) + 1][cc % NS] : sb;
+          sa = mine ? s[2 * (cc / G)][cc % G] : sa;
+          sb = mine ? s[2 * (cc / G) + 1][cc % G] : sb;
         } else {
-          sa = mine ? s[cc / NS][cc % NS] : sa;
+          sa = mine ? s[cc / G][cc % G] : sa;
         }
       }
-      const int g = SPLIT ? gq0 + c % NS : c % G;
-      const int jl = SPLIT ? c % NS : g;  // its slot in lsum
+      const int g = c % G;
 #pragma unroll
       for (int gg = 0; gg < G; ++gg) mc = g == gg ? mneg[gg] : mc;
       if constexpr (HALF) {
         const float pa = fast_exp2(fmaf(sa, scale, mc));
         const float pb = fast_exp2(fmaf(sb, scale, mc));
 #pragma unroll
-        for (int gg = 0; gg < NS; ++gg) lsum[gg] += jl == gg ? pa + pb : 0.f;
-        sp[((c / NS) * GPW + gi) * G + g] = pack_half2<T>(pa, pb);
+        for (int gg = 0; gg < G; ++gg) lsum[gg] += g == gg ? pa + pb : 0.f;
+        sp[((c / G) * GPW + gi) * G + g] = pack_half2<T>(pa, pb);
       } else {
         const float pa = fast_exp2(fmaf(sa, scale, mc));
 #pragma unroll
-        for (int gg = 0; gg < NS; ++gg) lsum[gg] += jl == gg ? pa : 0.f;
-        sp[(gi + GPW * (c / NS)) * G + g] = __float_as_uint(pa);
+        for (int gg = 0; gg < G; ++gg) lsum[gg] += g == gg ? pa : 0.f;
+        sp[(gi + GPW * (c / G)) * G + g] = __float_as_uint(pa);
       }
     }
     __builtin_amdgcn_wave_barrier();
@@ -821,9 +742,9 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
         if (((R * u) % (2 * GPW)) >= GPW) continue;
         const int t = R * u + sub;
         const int pidx = (t / (2 * GPW)) * GPW + (t % GPW);
-        uint32_t pw[GA];
+        uint32_t pw[G];
 #pragma unroll
-        for (int j = 0; j < GA; ++j) pw[j] = sp[pidx * G + (PAIR ? hh * GA + j : j)];
+        for (int j = 0; j < G; ++j) pw[j] = sp[pidx * G + j];
 #pragma unroll
         for (int w = 0; w < PE / 2; ++w) {
           // Element 2w (lo) and 2w+1 (hi) of tokens t and t + GPW, paired.
@@ -831,7 +752,7 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
           const uint32_t lo = __builtin_amdgcn_perm(vbb, va, 0x05040100u);
           const uint32_t hi = __builtin_amdgcn_perm(vbb, va, 0x07060302u);
 #pragma unroll
-          for (int j = 0; j < GA; ++j) {
+          for (int j = 0; j < G; ++j) {
             acc[j][2 * w] = dot2_half<T>(pw[j], lo, acc[j][2 * w]);
             acc[j][2 * w + 1] = dot2_half<T>(pw[j], hi, acc[j][2 * w + 1]);
           }
@@ -849,7 +770,7 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
           v[1] = __uint_as_float(vb[u].y);
         }
 #pragma unroll
-        for (int g = 0; g < GA; ++g) {
+        for (int g = 0; g < G; ++g) {
           const float p = __uint_as_float(sp[t * G + g]);
 #pragma unroll
           for (int e = 0; e < PE; ++e) acc[g][e] = fmaf(p, v[e], acc[g][e]);
@@ -900,9 +821,7 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
   float ltot[G];
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    float l = SPLIT ? (khalf == g / GA ? lsum[g % NS] : 0.f)
-              : RS  ? (lig == g / HPL ? lsum[g % HPL] : 0.f)
-                    : lsum[g % NS];
+    float l = RS ? (lig == g / HPL ? lsum[g % HPL] : 0.f) : lsum[g];
 #pragma unroll
     for (int o = kWave / 2; o >= 1; o >>= 1) l += __shfl_xor(l, o, kWave);
     ltot[g] = l;
@@ -911,18 +830,14 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
 #pragma unroll
   for (int o = kWave / 2; o >= S::kLp; o >>= 1)
 #pragma unroll
-    for (int j = 0; j < GA; ++j)
+    for (int j = 0; j < G; ++j)
 #pragma unroll
       for (int e = 0; e < PE; ++e) acc[j][e] += __shfl_xor(acc[j][e], o, kWave);
   if (sub == 0) {
-    // s_acc rows hold OUT_D elements: when paired, the half of the row that
-    // belongs to the head's own real KV head (the lane's slice lies in the
-    // half of real head hh, whose query heads are hh*GA .. hh*GA + GA-1).
 #pragma unroll
-    for (int j = 0; j < GA; ++j)
+    for (int j = 0; j < G; ++j)
 #pragma unroll
-      for (int e = 0; e < PE; ++e)
-        s_acc[wave][(PAIR ? hh * GA + j : j) * OUT_D + lp * PE - hh * OUT_D + e] = acc[j][e];
+      for (int e = 0; e < PE; ++e) s_acc[wave][j * D + lp * PE + e] = acc[j][e];
   }
   if (lane < G) {
 #pragma unroll
@@ -934,16 +849,14 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
   }
   __syncthreads();
 
-  // Outputs and partials use the real layout [.., H_q, OUT_D]: this
-  // workgroup's G query heads are the real heads h0 .. h0 + G-1 (for a pair,
-  // those of both of its KV heads).
+  // This workgroup's G query heads are h0 .. h0 + G-1.
   const int hq = hkv * a.group;
   const int nparts = (ctx + a.partition - 1) / a.partition;
-  float* pacc = a.part_acc + (item * hq + h0) * ODM;
-  T* out = reinterpret_cast<T*>(a.output) + (qtok * hq + h0) * ODM;
-  for (int i = tid; i < G * ODM; i += kDecodeThreads) {
-    const int g = i / ODM;
-    const int si = MASKD ? g * OUT_D + (i - g * ODM) : i;  // its s_acc element
+  float* pacc = a.part_acc + (item * hq + h0) * DM;
+  T* out = reinterpret_cast<T*>(a.output) + (qtok * hq + h0) * DM;
+  for (int i = tid; i < G * DM; i += kDecodeThreads) {
+    const int g = i / DM;
+    const int si = MASKD ? g * D + (i - g * DM) : i;  // its s_acc element
     float mx = s_m[0][g];
 #pragma unroll
     for (int w = 1; w < kDecodeWaves; ++w) mx = fmaxf(mx, s_m[w][g]);
@@ -958,7 +871,7 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
       store_scalar<T>(out + i, l > 0.f ? o / l : 0.f);
     } else {
       store_device(pacc + i, o);
-      if (i % ODM == 0) {
+      if (i % DM == 0) {
         float* pml = a.part_ml + (item * hq + h0 + g) * 2;
         store_device(pml, mx);
         store_device(pml + 1, l);
@@ -970,12 +883,12 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, (PAIR ? G
   if (nparts > 1 && n > 0 && a.merge_state != nullptr && seq >= 0 && seq < a.num_seqs) {
     // (fp32 heads of 80 and 96 merge one element at a time, which keeps
     // their occupancy.)
-    constexpr int KO = (G * ODM + kDecodeThreads - 1) / kDecodeThreads;
+    constexpr int KO = (G * DM + kDecodeThreads - 1) / kDecodeThreads;
     constexpr int KM = MASKD && sizeof(T) == 4 ? 1 : kMergeOutputs;
     constexpr int KC = KO >= 4 && KM >= 4 ? 4 : KO >= 2 && KM >= 2 ? 2 : 1;
-    merge_in_launch<T, ODM, KC>(a, G, part, item, ctx, nparts,
+    merge_in_launch<T, DM, KC>(a, G, part, item, ctx, nparts,
                                    (static_cast<int64_t>(seq) * hkv + kvh) * a.sub_groups + sg, h0, hq,
-                                   reinterpret_cast<T*>(a.output) + qtok * hq * ODM);
+                                   reinterpret_cast<T*>(a.output) + qtok * hq * DM);
   }
 }
 
@@ -1014,7 +927,7 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_merge_kernel(DecodeArgs
 // ---- host-side dispatch ------------------------------------------------
 
 // The merge phase, unless the partition launch merged in place (merge
-// records given): all a.group query heads of a KV head (or pair) merge in one
+// records given): all a.group query heads of a KV head merge in one
 // workgroup row; out_d: elements per query head in memory.
 template <typename T>
 static hipError_t launch_merge_t(const DecodeArgs& a, int out_d, int phases, hipStream_t stream) {
@@ -1034,120 +947,82 @@ static hipError_t launch_merge(const DecodeArgs& a, int dtype, int out_d, int ph
 }
 
 // Launches both phases of one kernel instance.  D, G: the kernel's head dim
-// and group (twice the real ones when paired).
+// and group.
 struct LaunchOp {
   const DecodeArgs& a;
   int64_t num_items;
   int phases;
   hipStream_t stream;
-  template <typename T, int D, int G, bool PAIR, bool SHARED, int DM>
+  template <typename T, int D, int G, bool SHARED, int DM>
   hipError_t run() const {
     const int64_t grid = num_items * a.num_kv_heads * a.sub_groups;
     if (phases & PA_DECODE_PHASE_PARTITIONS) {
-      hipLaunchKernelGGL((decode_partition_kernel<T, D, G, PAIR, SHARED, DM>), dim3(static_cast<uint32_t>(grid)),
+      hipLaunchKernelGGL((decode_partition_kernel<T, D, G, SHARED, DM>), dim3(static_cast<uint32_t>(grid)),
                          dim3(kDecodeThreads), 0, stream, a);
       const hipError_t err = hipGetLastError();
       if (err != hipSuccess) return err;
     }
-    // Partials are in the real layout: rows of D/2 when paired.
-    return launch_merge_t<T>(a, PAIR ? D / 2 : DM, phases, stream);
+    return launch_merge_t<T>(a, DM, phases, stream);
   }
 };
 
 // Resident partition workgroups per CU of one kernel instance.
 struct OccupancyOp {
   int* per_cu;
-  template <typename T, int D, int G, bool PAIR, bool SHARED, int DM>
+  template <typename T, int D, int G, bool SHARED, int DM>
   hipError_t run() const {
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, decode_partition_kernel<T, D, G, PAIR, SHARED, DM>,
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, decode_partition_kernel<T, D, G, SHARED, DM>,
                                                         kDecodeThreads, 0);
   }
 };
 
-template <typename T, int D, int G, bool PAIR, bool SHARED, int DM, typename Op>
-static hipError_t visit_one(const Op& op) {
-  if constexpr (PAIR && G % 2 != 0) {
-    return hipErrorNotSupported;  // a pair's group is even
-  } else {
-    return op.template run<T, D, G, PAIR, SHARED, DM>();
-  }
-}
-
-template <typename T, int D, bool PAIR, bool SHARED = false, int DM = D, typename Op>
+template <typename T, int D, bool SHARED, int DM, typename Op>
 static hipError_t visit_group(int G, const Op& op) {
   switch (G) {
-    case 1: return visit_one<T, D, 1, PAIR, SHARED, DM>(op);
-    case 2: return visit_one<T, D, 2, PAIR, SHARED, DM>(op);
-    case 3: return visit_one<T, D, 3, PAIR, SHARED, DM>(op);
-    case 4: return visit_one<T, D, 4, PAIR, SHARED, DM>(op);
-    case 5: return visit_one<T, D, 5, PAIR, SHARED, DM>(op);
-    case 6: return visit_one<T, D, 6, PAIR, SHARED, DM>(op);
-    case 7: return visit_one<T, D, 7, PAIR, SHARED, DM>(op);
-    case 8: return visit_one<T, D, 8, PAIR, SHARED, DM>(op);
+    case 1: return op.template run<T, D, 1, SHARED, DM>();
+    case 2: return op.template run<T, D, 2, SHARED, DM>();
+    case 3: return op.template run<T, D, 3, SHARED, DM>();
+    case 4: return op.template run<T, D, 4, SHARED, DM>();
+    case 5: return op.template run<T, D, 5, SHARED, DM>();
+    case 6: return op.template run<T, D, 6, SHARED, DM>();
+    case 7: return op.template run<T, D, 7, SHARED, DM>();
+    case 8: return op.template run<T, D, 8, SHARED, DM>();
     default: return hipErrorNotSupported;
   }
 }
 
 template <bool SHARED, typename Op>
-static hipError_t visit_unpaired(int dtype, int head_dim, int g, const Op& op) {
+static hipError_t visit_shape(int dtype, int head_dim, int g, const Op& op) {
   if (dtype == PA_DTYPE_BF16) {
-    if (head_dim == 256) return visit_group<bf16_t, 256, false, SHARED>(g, op);
-    if (head_dim == 96) return visit_group<bf16_t, 128, false, SHARED, 96>(g, op);
-    if (head_dim == 80) return visit_group<bf16_t, 128, false, SHARED, 80>(g, op);
+    if (head_dim == 256) return visit_group<bf16_t, 256, SHARED, 256>(g, op);
+    if (head_dim == 96) return visit_group<bf16_t, 128, SHARED, 96>(g, op);
+    if (head_dim == 80) return visit_group<bf16_t, 128, SHARED, 80>(g, op);
   } else if (dtype == PA_DTYPE_F16) {
-    if (head_dim == 256) return visit_group<f16_t, 256, false, SHARED>(g, op);
-    if (head_dim == 96) return visit_group<f16_t, 128, false, SHARED, 96>(g, op);
-    if (head_dim == 80) return visit_group<f16_t, 128, false, SHARED, 80>(g, op);
+    if (head_dim == 256) return visit_group<f16_t, 256, SHARED, 256>(g, op);
+    if (head_dim == 96) return visit_group<f16_t, 128, SHARED, 96>(g, op);
+    if (head_dim == 80) return visit_group<f16_t, 128, SHARED, 80>(g, op);
   } else if (dtype == PA_DTYPE_F32) {
-    if (head_dim == 128) return visit_group<float, 128, false, SHARED>(g, op);
-    if (head_dim == 64) return visit_group<float, 64, false, SHARED>(g, op);
-    if (head_dim == 96) return visit_group<float, 128, false, SHARED, 96>(g, op);
-    if (head_dim == 80) return visit_group<float, 128, false, SHARED, 80>(g, op);
+    if (head_dim == 128) return visit_group<float, 128, SHARED, 128>(g, op);
+    if (head_dim == 64) return visit_group<float, 64, SHARED, 64>(g, op);
+    if (head_dim == 96) return visit_group<float, 128, SHARED, 96>(g, op);
+    if (head_dim == 80) return visit_group<float, 128, SHARED, 80>(g, op);
   }
   return hipErrorNotSupported;
 }
 
-// The kernel instance of a real shape: paired heads of D run as the
-// instance of head dim 2D and group 2G; a group above the largest kernel
-// group runs as decode_sub_groups(group) workgroups per KV head, on the
-// SHARED instances (cached K/V loads: the siblings' re-reads hit L2).
+// The kernel instance of a shape: a group above the largest kernel group
+// runs as decode_sub_groups(group) workgroups per KV head, on the SHARED
+// instances (cached K/V loads: the siblings' re-reads hit L2).
 template <typename Op>
-static hipError_t visit_decode(int dtype, int head_dim, int group, bool pair, const Op& op) {
-  if (pair) {
-    if (group < 1 || group > 4) return hipErrorNotSupported;
-    if (dtype == PA_DTYPE_BF16) {
-      if (head_dim == 64) return visit_group<bf16_t, 128, true>(2 * group, op);
-      if (head_dim == 128) return visit_group<bf16_t, 256, true>(2 * group, op);
-    } else if (dtype == PA_DTYPE_F16) {
-      if (head_dim == 64) return visit_group<f16_t, 128, true>(2 * group, op);
-      if (head_dim == 128) return visit_group<f16_t, 256, true>(2 * group, op);
-    }
-    return hipErrorNotSupported;
-  }
+static hipError_t visit_decode(int dtype, int head_dim, int group, const Op& op) {
   if (group < 1) return hipErrorNotSupported;
   const int nsub = decode_sub_groups(group);
-  return nsub > 1 ? visit_unpaired<true>(dtype, head_dim, group / nsub, op)
-                  : visit_unpaired<false>(dtype, head_dim, group, op);
+  return nsub > 1 ? visit_shape<true>(dtype, head_dim, group / nsub, op)
+                  : visit_shape<false>(dtype, head_dim, group, op);
 }
 
-// Largest real group run as pairs, per real head dim (bf16 and fp16; 0 = never).
-// Kernel time on 256 lognormal contexts (median 1024) with 8 KV heads,
-// unpaired -> paired, each at its best partition:
-//   D 64:  G 1 0.180 -> 0.141 ms, G 2 0.181 -> 0.140, G 3 0.183 -> 0.147,
-//          G 4 0.183 -> 0.149;
-//   D 128: G 1 0.267 -> 0.253, G 2 0.267 -> 0.259, G 3 0.269 -> 0.261,
-//          G 4 0.271 -> 0.267 (three waves per SIMD: the eight heads' state
-//          does not fit the register budget of four without spilling).
-#ifndef PA_DECODE_PAIR_MAX_GROUP_D64
-#define PA_DECODE_PAIR_MAX_GROUP_D64 4
-#endif
-#ifndef PA_DECODE_PAIR_MAX_GROUP_D128
-#define PA_DECODE_PAIR_MAX_GROUP_D128 4
-#endif
-
 int decode_unit_heads(int dtype, int head_dim, int num_kv_heads, int group) {
-  if (!decode_uses_mfma(dtype, head_dim) || num_kv_heads % 2 != 0 || group < 1) return 1;
-  return group <= (head_dim == 64 ? PA_DECODE_PAIR_MAX_GROUP_D64 : PA_DECODE_PAIR_MAX_GROUP_D128) ? 2 : 1;
+  return decode_uses_mfma(dtype, head_dim) && num_kv_heads % 2 == 0 && group >= 1 && group <= 4 ? 2 : 1;
 }
 
 int decode_sub_groups(int group) {
@@ -1180,32 +1055,25 @@ bool decode_fast_path_supported(int dtype, int head_dim, int group, int block_si
 hipError_t launch_decode(const DecodeArgs& a, int dtype, int head_dim, int group,
                          int64_t num_items, int phases, hipStream_t stream) {
   if (num_items <= 0) return hipSuccess;
-  if (decode_unit_heads(dtype, head_dim, a.num_kv_heads, group) == 2) {
-    DecodeArgs p = a;
-    p.num_kv_heads = a.num_kv_heads / 2;
-    p.group = 2 * a.group;
-    return visit_decode(dtype, head_dim, group, true, LaunchOp{p, num_items, phases, stream});
-  }
   if (decode_uses_mfma(dtype, head_dim)) {
     if (phases & PA_DECODE_PHASE_PARTITIONS) {
-      const hipError_t err = launch_decode_mfma(a, dtype, head_dim, num_items, stream);
+      const int heads = decode_unit_heads(dtype, head_dim, a.num_kv_heads, group);
+      const hipError_t err = launch_decode_mfma(a, dtype, head_dim, heads, num_items, stream);
       if (err != hipSuccess) return err;
     }
     return launch_merge(a, dtype, head_dim, phases, stream);
   }
-  return visit_decode(dtype, head_dim, group, false, LaunchOp{a, num_items, phases, stream});
+  return visit_decode(dtype, head_dim, group, LaunchOp{a, num_items, phases, stream});
 }
 
 hipError_t decode_workgroups_per_cu(int dtype, int head_dim, int num_kv_heads, int group, int* per_cu) {
   *per_cu = 0;
-  const bool pair = decode_unit_heads(dtype, head_dim, num_kv_heads, group) == 2;
-  if (!pair && decode_uses_mfma(dtype, head_dim)) {
-    const int wgs = decode_workgroups_per_head(dtype, head_dim, group);
-    const hipError_t err = decode_mfma_workgroups_per_cu(dtype, head_dim, wgs > 1, per_cu);
-    *per_cu *= decode_sub_groups(group) / wgs;
-    return err;
-  }
-  return visit_decode(dtype, head_dim, group, pair, OccupancyOp{per_cu});
+  if (!decode_uses_mfma(dtype, head_dim)) return visit_decode(dtype, head_dim, group, OccupancyOp{per_cu});
+  const int wgs = decode_workgroups_per_head(dtype, head_dim, group);
+  const hipError_t err = decode_mfma_workgroups_per_cu(
+      dtype, head_dim, wgs > 1, decode_unit_heads(dtype, head_dim, num_kv_heads, group), per_cu);
+  *per_cu *= decode_sub_groups(group) / wgs;
+  return err;
 }
 
 }  // namespace pa

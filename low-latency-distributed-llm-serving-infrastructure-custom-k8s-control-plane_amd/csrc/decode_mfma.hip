@@ -1,6 +1,7 @@
 // Paged-attention decode of 16-bit caches on the matrix cores: one workgroup
-// per (sequence, context partition, KV head), up to 16 query heads of the KV
-// head in one pass (larger groups run as sub-groups of at most 16).
+// per (sequence, context partition, KV head or two adjacent ones), up to 16
+// query heads of a KV head in one pass (larger groups run as sub-groups of at
+// most 16).
 //
 // What bounds it is HBM: every K/V byte is read once for all 16 heads, and a
 // 32-token tile costs a wave 16 MFMAs and about 100 vector instructions
@@ -33,7 +34,14 @@
 // K as operand loads straight from HBM (64 bytes of 16 rows an instruction,
 // no LDS) took 164 us in the first of those steps; streaming (nontemporal)
 // loads are worth 11-13 % where no sibling reads the rows again.
-// Each wave runs its own online softmax over every fourth tile, the next
+// HEADS 2 (groups of up to 4, an even KV head count): half of the waves take
+// each of two adjacent KV heads, so that both halves of a token's 512 (or 256)
+// contiguous bytes are read by one workgroup at about the same time.  Against
+// the vector kernel that read them as one row: 256 sequences of 32-8192
+// tokens, 32/8 heads of 128, 268 -> 258 us (6.6 TB/s), 64 sequences, 32/32
+// heads, 343 -> 341; one workgroup per head took 274 and 356.
+// Each wave runs its own online softmax over every fourth tile (every second
+// one of its head's with HEADS 2), the next
 // tile's K and V loads in flight under the current tile's arithmetic, no
 // barrier in the loop.
 #include "decode_common.hpp"
@@ -80,7 +88,7 @@ __device__ __forceinline__ V row_load(const void* p) {
   return *reinterpret_cast<const V*>(p);
 }
 
-template <typename T, int D, bool SHARED>
+template <typename T, int D, bool SHARED, int HEADS>
 __global__ __launch_bounds__(kDecodeThreads) __attribute__((amdgpu_waves_per_eu(3))) void
 decode_mfma_kernel(DecodeArgs a) {
   static_assert(sizeof(T) == 2, "16-bit caches");
@@ -105,6 +113,7 @@ decode_mfma_kernel(DecodeArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int r = lane & 15;  // token of a K load, query head elsewhere
   const int c = lane >> 4;
+  constexpr int kHeadWaves = kDecodeWaves / HEADS;  // waves per KV head
   const int hkv = a.num_kv_heads;
   const int G = a.group / a.sub_groups;
   // Workgroup -> (item, KV head, sub-group).  Ids are dealt to the XCDs
@@ -113,19 +122,21 @@ decode_mfma_kernel(DecodeArgs a) {
   // 8 gangs, the last may be shorter).  Sub-groups that read the same rows
   // form a gang, whose later reads hit that XCD's L2; so do all of an item's
   // heads of 64, whose rows of 128 bytes share HBM bursts (128 sequences, 16/8
-  // heads: 208 -> 196 us), but not its heads of 128 (64 sequences, 32/32
-  // heads: 344 us spread over the XCDs, 357 as one gang).
-  const int gang_heads = D == 64 ? hkv : 1;
+  // heads: 208 -> 196 us), but not its heads of 128 (256 sequences, 32/8 heads:
+  // 258 us spread over the XCDs, 265 as one gang).
+  const int units = hkv / HEADS;
+  const int gang_heads = D == 64 ? units : 1;
   const int gang = gang_heads * a.sub_groups;
   const int64_t run = blockIdx.x / (kXcds * gang);
   const int at_run = static_cast<int>(blockIdx.x - run * (kXcds * gang));
   const int width = static_cast<int>(min<int64_t>(kXcds, gridDim.x / gang - run * kXcds));
   const int member = at_run / width;
   const int64_t g_id = run * kXcds + (at_run - member * width);
-  const int64_t item = g_id / (hkv / gang_heads);
-  const int kvh = static_cast<int>(g_id - item * (hkv / gang_heads)) * gang_heads + member / a.sub_groups;
+  const int64_t item = g_id / (units / gang_heads);
+  const int unit = static_cast<int>(g_id - item * (units / gang_heads)) * gang_heads + member / a.sub_groups;
+  const int kvh = unit * HEADS + wave / kHeadWaves;
   const int sg = member % a.sub_groups;
-  const int h0 = kvh * a.group + sg * G;  // first query head
+  const int h0 = kvh * a.group + sg * G;  // first query head of the wave
   const int seq = a.items[2 * item];
   const int part = a.items[2 * item + 1];
   const int64_t trow = a.rows != nullptr ? a.rows[seq] : seq;
@@ -171,7 +182,7 @@ decode_mfma_kernel(DecodeArgs a) {
   constexpr int kAppendPieces = kRowBytes / 16;
   const int ntiles = (n + kMfmaTile - 1) / kMfmaTile;
   const bool append = a.new_key != nullptr && n > 0 && p0 + n == ctx;
-  const bool append_wave = append && (ntiles - 1) % kDecodeWaves == wave;
+  const bool append_wave = append && (ntiles - 1) % kHeadWaves == wave % kHeadWaves;
   char* append_dst = nullptr;
   uint4 append_piece = make_uint4(0, 0, 0, 0);
   if (append_wave && lane < 2 * kAppendPieces) {
@@ -343,10 +354,10 @@ decode_mfma_kernel(DecodeArgs a) {
     }
   };
 
-  if (wave < ntiles) {
-    int tile = wave;
+  if (wave % kHeadWaves < ntiles) {
+    int tile = wave % kHeadWaves;
     if (log2_bs < 4 || hole) {
-      for (; tile < ntiles; tile += kDecodeWaves) {
+      for (; tile < ntiles; tile += kHeadWaves) {
         write_new_rows(tile);
         load_any(tile);
         scores();
@@ -363,10 +374,10 @@ decode_mfma_kernel(DecodeArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       load_v();
       __builtin_amdgcn_sched_barrier(0);
-      for (; tile + kDecodeWaves < ntiles; tile += kDecodeWaves) {
-        locate(tile + kDecodeWaves);
+      for (; tile + kHeadWaves < ntiles; tile += kHeadWaves) {
+        locate(tile + kHeadWaves);
         scores();
-        write_new_rows(tile + kDecodeWaves);
+        write_new_rows(tile + kHeadWaves);
         __builtin_amdgcn_sched_barrier(0);
         load_k();
         __builtin_amdgcn_sched_barrier(0);
@@ -397,35 +408,38 @@ decode_mfma_kernel(DecodeArgs a) {
 
   const int hq = hkv * a.group;
   const int nparts = (ctx + a.partition - 1) / a.partition;
-  float* pacc = a.part_acc + (item * hq + h0) * D;
-  T* out = reinterpret_cast<T*>(a.output) + (qtok * hq + h0) * D;
-  for (int i = tid; i < G * D; i += kDecodeThreads) {
-    const int g = i / D;
-    const int e = g * kAccRow + (i - g * D);
-    float mx = s_m[0][g];
+  const int hu = unit * HEADS * a.group + sg * G;  // first query head of the workgroup
+  float* pacc = a.part_acc + (item * hq + hu) * D;
+  T* out = reinterpret_cast<T*>(a.output) + (qtok * hq + hu) * D;
+  for (int i = tid; i < HEADS * G * D; i += kDecodeThreads) {
+    const int hg = i / D;
+    const int w0 = HEADS == 1 ? 0 : hg / G * kHeadWaves;  // the head's first wave
+    const int g = HEADS == 1 ? hg : hg % G;
+    const int e = g * kAccRow + (i - hg * D);
+    float mx = s_m[w0][g];
 #pragma unroll
-    for (int w = 1; w < kDecodeWaves; ++w) mx = fmaxf(mx, s_m[w][g]);
+    for (int w = 1; w < kHeadWaves; ++w) mx = fmaxf(mx, s_m[w0 + w][g]);
     float o = 0.f, sum = 0.f;
 #pragma unroll
-    for (int w = 0; w < kDecodeWaves; ++w) {
-      const float f = fast_exp2(s_m[w][g] - mx);
-      o = fmaf(reinterpret_cast<const float*>(s_wave[w])[e], f, o);
-      sum = fmaf(s_l[w][g], f, sum);
+    for (int w = 0; w < kHeadWaves; ++w) {
+      const float f = fast_exp2(s_m[w0 + w][g] - mx);
+      o = fmaf(reinterpret_cast<const float*>(s_wave[w0 + w])[e], f, o);
+      sum = fmaf(s_l[w0 + w][g], f, sum);
     }
     if (nparts <= 1) {
       store_scalar<T>(out + i, sum > 0.f ? o / sum : 0.f);
     } else {
       store_device(pacc + i, o);
       if (i % D == 0) {
-        float* pml = a.part_ml + (item * hq + h0 + g) * 2;
+        float* pml = a.part_ml + (item * hq + hu + hg) * 2;
         store_device(pml, mx);
         store_device(pml + 1, sum);
       }
     }
   }
   if (nparts > 1 && n > 0 && a.merge_state != nullptr && seq >= 0 && seq < a.num_seqs)
-    merge_in_launch<T, D, kMergeOutputs>(a, G, part, item, ctx, nparts,
-                                         (static_cast<int64_t>(seq) * hkv + kvh) * a.sub_groups + sg, h0, hq,
+    merge_in_launch<T, D, kMergeOutputs>(a, HEADS * G, part, item, ctx, nparts,
+                                         (static_cast<int64_t>(seq) * units + unit) * a.sub_groups + sg, hu, hq,
                                          reinterpret_cast<T*>(a.output) + qtok * hq * D);
 }
 
@@ -433,14 +447,20 @@ bool decode_uses_mfma(int dtype, int head_dim) {
   return (dtype == PA_DTYPE_BF16 || dtype == PA_DTYPE_F16) && (head_dim == 64 || head_dim == 128);
 }
 
+template <typename T, int D, typename Op>
+static hipError_t visit_mfma_t(bool shared, int heads, const Op& op) {
+  if (heads == 2) return op.template run<T, D, false, 2>();
+  return shared ? op.template run<T, D, true, 1>() : op.template run<T, D, false, 1>();
+}
+
 template <typename Op>
-static hipError_t visit_mfma(int dtype, int head_dim, bool shared, const Op& op) {
+static hipError_t visit_mfma(int dtype, int head_dim, bool shared, int heads, const Op& op) {
   if (dtype == PA_DTYPE_BF16) {
-    if (head_dim == 128) return shared ? op.template run<bf16_t, 128, true>() : op.template run<bf16_t, 128, false>();
-    if (head_dim == 64) return shared ? op.template run<bf16_t, 64, true>() : op.template run<bf16_t, 64, false>();
+    if (head_dim == 128) return visit_mfma_t<bf16_t, 128>(shared, heads, op);
+    if (head_dim == 64) return visit_mfma_t<bf16_t, 64>(shared, heads, op);
   } else if (dtype == PA_DTYPE_F16) {
-    if (head_dim == 128) return shared ? op.template run<f16_t, 128, true>() : op.template run<f16_t, 128, false>();
-    if (head_dim == 64) return shared ? op.template run<f16_t, 64, true>() : op.template run<f16_t, 64, false>();
+    if (head_dim == 128) return visit_mfma_t<f16_t, 128>(shared, heads, op);
+    if (head_dim == 64) return visit_mfma_t<f16_t, 64>(shared, heads, op);
   }
   return hipErrorNotSupported;
 }
@@ -449,29 +469,31 @@ struct MfmaLaunch {
   const DecodeArgs& a;
   int64_t num_items;
   hipStream_t stream;
-  template <typename T, int D, bool SHARED>
+  template <typename T, int D, bool SHARED, int HEADS>
   hipError_t run() const {
-    const int64_t grid = num_items * a.num_kv_heads * a.sub_groups;
-    hipLaunchKernelGGL((decode_mfma_kernel<T, D, SHARED>), dim3(static_cast<uint32_t>(grid)), dim3(kDecodeThreads), 0,
-                       stream, a);
+    const int64_t grid = num_items * (a.num_kv_heads / HEADS) * a.sub_groups;
+    hipLaunchKernelGGL((decode_mfma_kernel<T, D, SHARED, HEADS>), dim3(static_cast<uint32_t>(grid)),
+                       dim3(kDecodeThreads), 0, stream, a);
     return hipGetLastError();
   }
 };
 
 struct MfmaOccupancy {
   int* per_cu;
-  template <typename T, int D, bool SHARED>
+  template <typename T, int D, bool SHARED, int HEADS>
   hipError_t run() const {
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, decode_mfma_kernel<T, D, SHARED>, kDecodeThreads, 0);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, decode_mfma_kernel<T, D, SHARED, HEADS>,
+                                                        kDecodeThreads, 0);
   }
 };
 
-hipError_t launch_decode_mfma(const DecodeArgs& a, int dtype, int head_dim, int64_t num_items, hipStream_t stream) {
-  return visit_mfma(dtype, head_dim, a.sub_groups > 1, MfmaLaunch{a, num_items, stream});
+hipError_t launch_decode_mfma(const DecodeArgs& a, int dtype, int head_dim, int unit_heads, int64_t num_items,
+                              hipStream_t stream) {
+  return visit_mfma(dtype, head_dim, a.sub_groups > 1, unit_heads, MfmaLaunch{a, num_items, stream});
 }
 
-hipError_t decode_mfma_workgroups_per_cu(int dtype, int head_dim, bool shared, int* per_cu) {
-  return visit_mfma(dtype, head_dim, shared, MfmaOccupancy{per_cu});
+hipError_t decode_mfma_workgroups_per_cu(int dtype, int head_dim, bool shared, int unit_heads, int* per_cu) {
+  return visit_mfma(dtype, head_dim, shared, unit_heads, MfmaOccupancy{per_cu});
 }
 
 }  // namespace pa
