@@ -43,6 +43,7 @@ EXPORTED_SYMBOLS = (
     "pa_pack_workspace_size",
     "pa_pack",
     "pa_plan_step",
+    "pa_plan_step_for",
     "pa_reshape_and_cache",
     "pa_copy_blocks",
     "pa_swap_blocks",
@@ -179,6 +180,7 @@ _SIGNATURES = {
          _vp, _sz, _vp, _sz, _vp],
     ),
     "pa_plan_step": (ctypes.c_int, [_vp, _vp, _vp, _i32, PaPlanParams, ctypes.POINTER(PaStepPlan)]),
+    "pa_plan_step_for": (ctypes.c_int, [_vp, _vp, _vp, _i32, PaPlanParams, _i32, _i32, ctypes.POINTER(PaStepPlan)]),
     "pa_calibrate_mfma": (ctypes.c_int, [_vp, _i32, _i32, _i32, _vp]),
     "pa_calibrate_mfma_flops": (ctypes.c_int64, [_i32, _i32]),
     "pa_calibrate_read": (ctypes.c_int, [_vp, _i64, _vp, _i32, _vp]),

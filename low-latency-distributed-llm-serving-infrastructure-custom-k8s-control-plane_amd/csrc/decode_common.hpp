@@ -161,7 +161,6 @@ __device__ __forceinline__ void merge_in_launch(const DecodeArgs& a, int G, int 
 }
 
 // decode_mfma.hip
-bool decode_uses_mfma(int dtype, int head_dim);
 hipError_t launch_decode_mfma(const DecodeArgs& a, int dtype, int head_dim, int unit_heads, int64_t num_items, hipStream_t stream);
 hipError_t decode_mfma_workgroups_per_cu(int dtype, int head_dim, bool shared, int unit_heads, int* per_cu);
 

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "decode_shape.hpp"
+
 namespace pa {
 
 // Decode (split-K) over block tables.
@@ -206,18 +208,6 @@ bool decode_fast_path_supported(int dtype, int head_dim, int group, int block_si
 // Largest query-head group the decode serves (split into sub-groups of at
 // most 8 heads above 8).
 constexpr int kMaxDecodeQueryGroup = 64;
-// Workgroups sharing one KV head's query heads: the fewest equal sub-groups
-// of at most 8 heads.
-int decode_sub_groups(int group);
-// Workgroups one KV head's query heads take in the decode launch: the
-// sub-groups, or fewer where the matrix-core kernel serves up to 16 heads a
-// workgroup (the unit count stays that of the sub-groups).
-int decode_workgroups_per_head(int dtype, int head_dim, int group);
-// Adjacent KV heads that run as one workgroup: 2 for 16-bit heads of 64 and
-// 128 in groups of up to 4 with an even KV head count, else 1.  Such units are
-// what pa_decode_workgroups_per_item counts (times the sub-groups) and what
-// merge records are kept for.
-int decode_unit_heads(int dtype, int head_dim, int num_kv_heads, int group);
 // phases: PA_DECODE_PHASE_PARTITIONS and/or PA_DECODE_PHASE_MERGE;
 // head_dim and group are the model's.
 hipError_t launch_decode(const DecodeArgs& a, int dtype, int head_dim, int group,

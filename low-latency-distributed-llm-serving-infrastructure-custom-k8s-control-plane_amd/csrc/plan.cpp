@@ -6,6 +6,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include "decode_shape.hpp"
 #include "pa_error.hpp"
 #include "paged_attention_amd.h"
 
@@ -78,6 +79,59 @@ int64_t choose_partition(const DecodeContexts& d, const PaPlanParams& p, int64_t
   return best;
 }
 
+// The same for the matrix-core decode kernel (decode_mfma.hip), whose
+// workgroup alone reads 44 GB/s.  A launch that fills the chip at 1024 tokens
+// or more keeps the rule above (its picks are within 2 % of the best).  The
+// model of the others, fitted to 22 graph-replayed steps of 1-64 sequences of
+// 16-16384 tokens (its picks are the fastest power of two on 18 of them and
+// within 6 % on all; the model above lost up to 34 %, 64 sequences of 300-700
+// tokens at 64 instead of 1024: 36.6 against 27.5 us):
+//   read   the step's bytes at 6.45 TB/s, or the largest workgroup's at its own
+//          rate if that takes longer;
+//   launch 0.003 us per workgroup (its prologue and partial stores);
+//   merge  1 us and 1 us more per batch of 8 partials of the longest sequence.
+constexpr double kMfmaBytesPerUs = 43.7e3;
+constexpr double kHbmBytesPerUs = 6.45e6;
+constexpr double kMfmaWorkgroupUs = 0.003;
+constexpr double kMfmaMergeUs = 0.96;
+constexpr double kMfmaMergeUsPerBatch = 0.99;
+constexpr int64_t kMinFullChipMfmaPartition = 1024;
+
+int64_t choose_partition_mfma(const DecodeContexts& d, const PaPlanParams& p, int dtype, int head_dim,
+                              int64_t longest) {
+  const int64_t rule = choose_partition(d, p, longest);
+  const int64_t hkv = p.num_kv_heads > 0 ? p.num_kv_heads : 1;
+  const int64_t hq = p.num_query_heads > 0 ? p.num_query_heads : 4 * hkv;
+  const int group = static_cast<int>(hq / hkv > 0 ? hq / hkv : 1);
+  const int64_t width = p.workgroups_per_item > 0 ? p.workgroups_per_item : hkv;
+  const int64_t unit_slots = (p.compute_units > 0 ? p.compute_units : 256) *
+                             (p.workgroups_per_cu > 0 ? p.workgroups_per_cu : 3);
+  if (rule >= kMinFullChipMfmaPartition && d.workgroups(rule, width) >= 3 * unit_slots / 2) return rule;
+  const int64_t tokens = d.workgroups(1, 1);
+  if (tokens == 0) return rule;
+  // Units that one workgroup serves (sub-groups of 8 heads run two to one).
+  const int64_t per_wg = pa::decode_sub_groups(group) / pa::decode_workgroups_per_head(dtype, head_dim, group);
+  const int heads = pa::decode_unit_heads(dtype, head_dim, static_cast<int>(hkv), group);
+  const double wg_row = 4.0 * head_dim * heads;  // K and V bytes of a token a workgroup reads
+  const double total_us = static_cast<double>(tokens) * 4.0 * head_dim * static_cast<double>(hkv) / kHbmBytesPerUs;
+  int64_t best = kMinPartition;
+  double best_us = -1.0;
+  for (int64_t part = kMinPartition; part <= kMaxPartition; part *= 2) {
+    const int64_t wgs = d.workgroups(part, width) / per_wg;
+    const double bytes = wg_row * static_cast<double>(part < longest ? part : longest);
+    const double read = bytes / kMfmaBytesPerUs > total_us ? bytes / kMfmaBytesPerUs : total_us;
+    const int64_t parts = ceil_div(longest, part);
+    const double merge =
+        parts > 1 ? kMfmaMergeUs + kMfmaMergeUsPerBatch * static_cast<double>(ceil_div(parts, kMergeBatch)) : 0.0;
+    const double us = read + kMfmaWorkgroupUs * static_cast<double>(wgs) + merge;
+    if (best_us < 0.0 || us < best_us * (1.0 - 1e-9)) {
+      best = part;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 int plan_fail(PaStepPlan* plan, int32_t seq, const char* what) {
   if (plan != nullptr) plan->bad_seq = seq;
   return pa::set_error(PA_ERR_INVALID_ARGUMENT, "pa_plan_step: %s", what);
@@ -89,6 +143,11 @@ extern "C" {
 
 int pa_plan_step(const int64_t* starts, const int64_t* counts, const int64_t* allocated, int32_t num_seqs,
                  PaPlanParams params, PaStepPlan* plan) {
+  return pa_plan_step_for(starts, counts, allocated, num_seqs, params, -1, 0, plan);
+}
+
+int pa_plan_step_for(const int64_t* starts, const int64_t* counts, const int64_t* allocated, int32_t num_seqs,
+                     PaPlanParams params, int32_t dtype, int32_t head_dim, PaStepPlan* plan) {
   if (plan == nullptr) return plan_fail(nullptr, -1, "plan must not be NULL");
   memset(plan, 0, sizeof(*plan));
   plan->bad_seq = -1;
@@ -130,7 +189,9 @@ int pa_plan_step(const int64_t* starts, const int64_t* counts, const int64_t* al
     return plan_fail(plan, -1, "a step's context tokens must stay below 2^31");
   const DecodeContexts d{starts, counts, num_seqs};
   const int64_t part = params.partition_size > 0 ? params.partition_size
-                                                 : choose_partition(d, params, longest_decode);
+                       : pa::decode_uses_mfma(dtype, head_dim)
+                           ? choose_partition_mfma(d, params, dtype, head_dim, longest_decode)
+                           : choose_partition(d, params, longest_decode);
   plan->partition_size = static_cast<int32_t>(part);
   for (int32_t i = 0; i < num_seqs; ++i) {
     if (counts[i] != 1) continue;

@@ -359,7 +359,7 @@ class PackedStep:
 
 def _plan(starts: np.ndarray, counts: np.ndarray, block_size: int, prefill_tile: int, partition_size: int,
           num_kv_heads: int, num_query_heads: int, workgroups_per_item: int, workgroups_per_cu: int,
-          compute_units: int, allocated: Optional[np.ndarray] = None):
+          compute_units: int, allocated: Optional[np.ndarray] = None, dtype: int = -1, head_dim: int = 0):
     lib = _native.load_library()
     params = _native.PaPlanParams(block_size=int(block_size), prefill_tile=int(prefill_tile),
                                   partition_size=int(partition_size), num_kv_heads=int(num_kv_heads),
@@ -367,9 +367,9 @@ def _plan(starts: np.ndarray, counts: np.ndarray, block_size: int, prefill_tile:
                                   workgroups_per_item=int(workgroups_per_item),
                                   workgroups_per_cu=int(workgroups_per_cu), compute_units=int(compute_units))
     plan = _native.PaStepPlan()
-    status = lib.pa_plan_step(starts.ctypes.data, counts.ctypes.data,
-                              None if allocated is None else allocated.ctypes.data,
-                              int(starts.shape[0]), params, ctypes.byref(plan))
+    status = lib.pa_plan_step_for(starts.ctypes.data, counts.ctypes.data,
+                                  None if allocated is None else allocated.ctypes.data,
+                                  int(starts.shape[0]), params, dtype, head_dim, ctypes.byref(plan))
     if status != _native.PA_OK:
         if plan.bad_seq >= 0:
             raise ValueError(lib.pa_last_error_message().decode(errors="replace"))
@@ -636,7 +636,7 @@ def pack_step(
         per_cu = _occupancy_on(device, dtype, head_dim, num_kv_heads, hq)
     allocated = None if allocated_tokens is None else _int64_array(allocated_tokens)
     plan = _plan(starts, counts, block_size, prefill_tile, partition_size or 0, num_kv_heads, hq, per_item,
-                 per_cu, _compute_units(device), allocated)
+                 per_cu, _compute_units(device), allocated, dtype_code(dtype) if per_cu else -1, int(head_dim or 0))
     pooled = rows is not None
     n_upd = 0 if updates is None else int(updates.shape[0])
 

@@ -517,3 +517,30 @@ def test_append_tokens_equals_repeated_append_token():
                 tables.append((t.get_physical_blocks(), t.get_tokens_count(), pool.host.copy(), pool.tokens.copy()))
             (b1, n1, h1, k1), (b2, n2, h2, k2) = tables
             assert b1 == b2 and n1 == n2 and (h1 == h2).all() and (k1 == k2).all(), (start, n)
+
+
+@pytest.mark.parametrize("starts,heads,head_dim,want", [
+    ([511] * 64, (32, 8), 128, 512),        # 64 short contexts: one partition each, no merge
+    ([4095], (32, 8), 128, 128),            # one sequence: short partitions, several merge batches
+    ([16383], (32, 8), 128, 512),
+    ([8191] * 2, (64, 8), 128, 512),        # one KV head a workgroup
+    ([4095] * 4, (128, 8), 128, 512),       # 16 heads a workgroup, counted as two units
+    # fills the chip (4 units an item: 1024 at 4096, 2048 at 2048; 1152 wanted): the rule of pa_plan_step
+    ([3000] * 256, (32, 8), 128, 2048),
+])
+def test_partition_of_the_matrix_core_decode(starts, heads, head_dim, want):
+    """pa_plan_step_for: the matrix-core kernel's own model below a full chip,
+    pa_plan_step for any other shape and for a partition that is given."""
+    native = pkg("_native")
+    s, c = np.asarray(starts, dtype=np.int64), np.ones(len(starts), dtype=np.int64)
+    hq, hkv = heads
+    units = ops.decode_workgroups_per_item(torch.bfloat16, head_dim, hkv, hq)
+    per_cu = 6 if hq // hkv > 8 else 3
+
+    def plan(partition, dtype, dim):
+        return int(ops._plan(s, c, 16, 32, partition, hkv, hq, units, per_cu, 256, None, dtype, dim).partition_size)
+
+    assert plan(0, native.PA_DTYPE_BF16, head_dim) == want
+    assert plan(96, native.PA_DTYPE_BF16, head_dim) == 96
+    other = ops.choose_partition(starts, [1] * len(starts), hkv, hq, units, per_cu)
+    assert plan(0, native.PA_DTYPE_F32, head_dim) == plan(0, native.PA_DTYPE_BF16, 96) == plan(0, -1, 0) == other
