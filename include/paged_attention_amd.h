@@ -597,6 +597,43 @@ const char *pa_last_error_message(void);
 /* ABI version: bumped whenever a signature or a struct above changes. */
 int pa_abi_version(void);
 
+/* ---- (f) one layer of a packed step in one call -------------------------- */
+
+/* What a step's layers share: the launch arguments of pa_prefill, pa_decode
+ * and pa_reshape_and_cache for a step packed by pa_pack.  num_decode_items /
+ * num_prefill_items of 0: nothing of that kind. */
+typedef struct {
+    PaStepDims dims;
+    const int32_t *block_tables;
+    const int32_t *context_lens;
+    const int64_t *cu_seqlens;
+    const int32_t *decode_items;
+    int64_t num_decode_items;
+    const int32_t *merge_items;
+    int64_t num_merge_items;
+    const int32_t *prefill_items;
+    int64_t num_prefill_items;
+    const int64_t *scatter_slots; /* [dims.num_query_tokens] */
+    void *workspace;              /* pa_decode_workspace_size(dims, num_decode_items) */
+    size_t workspace_bytes;
+    int32_t prefill_tile;
+} PaStepCall;
+
+/* flags: write the multi-token sequences' new rows inside the prefill launch;
+ * write no rows inside the prefill and decode launches. */
+enum { PA_STEP_PREFILL_WRITE = 1, PA_STEP_NO_APPEND = 2 };
+
+/*
+ * One layer: writes the new rows into the caches and attends, as
+ * pa_prefill_append / pa_decode_append where their launches take the rows,
+ * else pa_reshape_and_cache ahead of pa_prefill and pa_decode.  A fused write
+ * that declines the shape (PA_ERR_UNSUPPORTED) sets *declined to 1 (0
+ * otherwise) and the rows are written by pa_reshape_and_cache.
+ */
+int pa_attention_step(const PaStepCall *call, const void *query, void *key_cache, void *value_cache,
+                      int32_t layer_idx, const PaNewRows *new_rows, float scaling, void *output,
+                      int32_t flags, int32_t *declined, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -33,6 +33,9 @@ PA_DECODE_PHASE_PARTITIONS = 1
 PA_DECODE_PHASE_MERGE = 2
 PA_DECODE_SCRATCH_BYTES = 64 << 20
 PA_DECODE_SCRATCH_STATE_BYTES = 1 << 20
+PA_STEP_PREFILL_WRITE = 1
+PA_STEP_NO_APPEND = 2
+
 PA_SWAP_OUT = 0
 PA_SWAP_IN = 1
 
@@ -58,6 +61,7 @@ EXPORTED_SYMBOLS = (
     "pa_decode_append",
     "pa_prefill",
     "pa_prefill_append",
+    "pa_attention_step",
     "pa_map_host_memory",
     "pa_calibrate_mfma",
     "pa_calibrate_mfma_flops",
@@ -134,6 +138,25 @@ class PaPackDims(ctypes.Structure):
     ]
 
 
+class PaStepCall(ctypes.Structure):
+    _fields_ = [
+        ("dims", PaStepDims),
+        ("block_tables", ctypes.c_void_p),
+        ("context_lens", ctypes.c_void_p),
+        ("cu_seqlens", ctypes.c_void_p),
+        ("decode_items", ctypes.c_void_p),
+        ("num_decode_items", ctypes.c_int64),
+        ("merge_items", ctypes.c_void_p),
+        ("num_merge_items", ctypes.c_int64),
+        ("prefill_items", ctypes.c_void_p),
+        ("num_prefill_items", ctypes.c_int64),
+        ("scatter_slots", ctypes.c_void_p),
+        ("workspace", ctypes.c_void_p),
+        ("workspace_bytes", ctypes.c_size_t),
+        ("prefill_tile", ctypes.c_int32),
+    ]
+
+
 class PaPlanParams(ctypes.Structure):
     _fields_ = [
         ("block_size", ctypes.c_int32),
@@ -178,6 +201,11 @@ _SIGNATURES = {
         ctypes.c_int,
         [_vp, _vp, _vp, _vp, _vp, PaPackDims, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
          _vp, _sz, _vp, _sz, _vp],
+    ),
+    "pa_attention_step": (
+        ctypes.c_int,
+        [ctypes.POINTER(PaStepCall), _vp, _vp, _vp, _i32, ctypes.POINTER(PaNewRows), ctypes.c_float, _vp, _i32,
+         ctypes.POINTER(_i32), _vp],
     ),
     "pa_plan_step": (ctypes.c_int, [_vp, _vp, _vp, _i32, PaPlanParams, ctypes.POINTER(PaStepPlan)]),
     "pa_plan_step_for": (ctypes.c_int, [_vp, _vp, _vp, _i32, PaPlanParams, _i32, _i32, ctypes.POINTER(PaStepPlan)]),

@@ -813,4 +813,59 @@ int pa_prefill_append(const void* query, void* key_cache, void* value_cache, int
                       output, stream, &new_rows);
 }
 
+int pa_attention_step(const PaStepCall* call, const void* query, void* key_cache, void* value_cache,
+                      int32_t layer_idx, const PaNewRows* new_rows, float scaling, void* output, int32_t flags,
+                      int32_t* declined, void* stream) {
+  int rc = require("pa_attention_step", {{call, "call"}, {new_rows, "new_rows"}, {declined, "declined"}});
+  if (rc != PA_OK) return rc;
+  *declined = 0;
+  const PaStepCall& c = *call;
+  bool prefill = c.num_prefill_items > 0, decode = c.num_decode_items > 0;
+  bool written = false;
+  if (!(flags & PA_STEP_NO_APPEND)) {
+    if (prefill && (flags & PA_STEP_PREFILL_WRITE)) {
+      rc = pa_prefill_append(query, key_cache, value_cache, layer_idx, c.dims, *new_rows, c.block_tables,
+                             c.context_lens, c.cu_seqlens, c.prefill_items, c.num_prefill_items, c.prefill_tile,
+                             scaling, output, stream);
+      if (rc != PA_OK && rc != PA_ERR_UNSUPPORTED) return rc;
+      if (rc == PA_OK) {
+        prefill = false;
+        written = true;
+      } else {
+        *declined = 1;
+      }
+    }
+    if (decode && !prefill) {
+      rc = pa_decode_append(query, key_cache, value_cache, layer_idx, c.dims, *new_rows, c.block_tables,
+                            c.context_lens, c.cu_seqlens, c.decode_items, c.num_decode_items, c.merge_items,
+                            c.num_merge_items, scaling, output, c.workspace, c.workspace_bytes, stream);
+      if (rc != PA_OK && rc != PA_ERR_UNSUPPORTED) return rc;
+      if (rc == PA_OK) {
+        decode = false;
+        written = true;
+      } else {
+        *declined = 1;
+      }
+    }
+  }
+  if (prefill || decode || !written) {
+    rc = pa_reshape_and_cache(new_rows->key, new_rows->value, new_rows->key_token_stride, new_rows->key_head_stride,
+                              new_rows->value_token_stride, new_rows->value_head_stride, key_cache, value_cache,
+                              c.scatter_slots, c.dims.num_query_tokens, c.dims.num_kv_heads, c.dims.head_dim,
+                              c.dims.block_size, c.dims.total_blocks, c.dims.num_layers, layer_idx, c.dims.dtype,
+                              stream);
+    if (rc != PA_OK) return rc;
+  }
+  if (prefill) {
+    rc = pa_prefill(query, key_cache, value_cache, layer_idx, c.dims, c.block_tables, c.context_lens, c.cu_seqlens,
+                    c.prefill_items, c.num_prefill_items, c.prefill_tile, scaling, output, stream);
+    if (rc != PA_OK) return rc;
+  }
+  if (decode)
+    return pa_decode(query, key_cache, value_cache, layer_idx, c.dims, c.block_tables, c.context_lens, c.cu_seqlens,
+                     c.decode_items, c.num_decode_items, c.merge_items, c.num_merge_items, scaling, output,
+                     c.workspace, c.workspace_bytes, stream);
+  return PA_OK;
+}
+
 }  // extern "C"

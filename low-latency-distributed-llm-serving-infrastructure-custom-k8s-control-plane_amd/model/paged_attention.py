@@ -146,7 +146,7 @@ class PagedStepContext:
 
     @property
     def num_query_tokens(self) -> int:
-        return int(self._counts.sum())
+        return int(self._counts.sum()) if self.packed is None else self.packed.num_query_tokens
 
     @property
     def num_context_tokens(self) -> int:

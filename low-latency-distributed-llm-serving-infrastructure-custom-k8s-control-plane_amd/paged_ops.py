@@ -17,6 +17,7 @@ plus :func:`attention` (decode + prefill of one flattened step) and
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Optional, Sequence, Tuple
 
 import numpy as np
@@ -40,7 +41,10 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """Handle of the current stream of ``device`` (its index, or the current
+    device's), without building a Stream object (4 us a call)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def _require_device(*tensors: torch.Tensor) -> torch.device:
@@ -48,7 +52,7 @@ def _require_device(*tensors: torch.Tensor) -> torch.device:
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 f"HIP paged-attention kernels need device tensors, got a tensor on {t.device}"
             )
@@ -68,8 +72,12 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 def prefill_tile_for(num_query_heads: int, num_kv_heads: int) -> int:
     """Query tokens per prefill work item: the tile the MFMA prefill kernel
     takes (128 query rows over one workgroup's heads; pa_prefill_tile)."""
-    lib = _native.load_library()
-    return int(lib.pa_prefill_tile(int(num_query_heads), int(num_kv_heads))) or 128
+    return _prefill_tile(int(num_query_heads), int(num_kv_heads))
+
+
+@functools.lru_cache(maxsize=256)
+def _prefill_tile(num_query_heads: int, num_kv_heads: int) -> int:
+    return int(_native.load_library().pa_prefill_tile(num_query_heads, num_kv_heads)) or 128
 
 
 # ---------------------------------------------------------------------------
@@ -94,11 +102,11 @@ class _Layout:
         self.nbytes = 0
 
     def add(self, name: str, dtype: torch.dtype, shape) -> None:
-        count = 1
+        size = _ELEM[dtype]
         for d in shape:
-            count *= d
+            size *= d
         self.fields[name] = (self.nbytes, dtype, shape)
-        self.nbytes += _align(count * _ELEM[dtype])
+        self.nbytes += (size + 255) & ~255
 
 
 class _HostStaging:
@@ -152,9 +160,12 @@ class _HostStaging:
             self._bufs[slot], self._arrays[slot], self._device[slot] = buf, buf.numpy(), int(dev.value)
         return slot, self._arrays[slot], self._device[slot]
 
-    def done(self, slot: int, stream) -> None:
-        """The launch reading ``slot`` is enqueued on ``stream``."""
-        self._streams[slot // self.HALF].setdefault(stream.cuda_stream, stream)
+    def done(self, slot: int, device: torch.device, handle: int) -> None:
+        """The launch reading ``slot`` is enqueued on ``device``'s current
+        stream, whose handle is ``handle``."""
+        streams = self._streams[slot // self.HALF]
+        if handle not in streams:
+            streams[handle] = torch.cuda.current_stream(device)
 
 
 _STAGING: dict = {}  # device -> _HostStaging
@@ -240,7 +251,9 @@ class PackedStep:
         count = 1
         for d in shape:
             count *= d
-        t = self.buffer[off : off + count * _ELEM[dtype]].view(dtype).view(shape)
+        t = self.buffer[off : off + count * _ELEM[dtype]].view(dtype)
+        if len(shape) != 1:
+            t = t.view(shape)
         self.__dict__[name] = t
         return t
 
@@ -406,9 +419,17 @@ def decode_workgroups_per_item(dtype: torch.dtype, head_dim: int, num_kv_heads: 
     """Partition workgroups the decode launches per work item: half the KV
     heads when adjacent heads run as pairs, KV heads x sub-groups for groups
     of more than 8 query heads, else the KV heads (0 for rejected counts)."""
-    lib = _native.load_library()
-    return int(lib.pa_decode_workgroups_per_item(dtype_code(dtype), int(head_dim), int(num_kv_heads),
-                                                 int(num_query_heads)))
+    return _workgroups_per_item(dtype_code(dtype), int(head_dim), int(num_kv_heads), int(num_query_heads))
+
+
+@functools.lru_cache(maxsize=256)
+def _workgroups_per_item(dtype: int, head_dim: int, num_kv_heads: int, num_query_heads: int) -> int:
+    return int(_native.load_library().pa_decode_workgroups_per_item(dtype, head_dim, num_kv_heads, num_query_heads))
+
+
+@functools.lru_cache(maxsize=1024)
+def _pack_workspace_size(num_seqs: int) -> int:
+    return int(_native.load_library().pa_pack_workspace_size(num_seqs))
 
 
 # (library, device, shape) -> workgroups per CU: the occupancy query is a
@@ -518,26 +539,29 @@ def _run_pack(step: PackedStep, with_gather: bool = False, updates: Optional[np.
         if n_upd:
             host[o_upd:nbytes].view(np.int32)[:] = updates.reshape(-1)
     table = step._source_table
-    step_table = step._layout.fields.get("block_tables")
-    dims = _native.PaPackDims(
-        num_seqs=b,
-        block_size=step.block_size,
-        max_blocks_per_seq=step.table_width,
-        partition_size=step.partition_size,
-        prefill_tile=step.prefill_tile,
-        num_table_rows=step._source_rows,
-        num_updates=n_upd,
-        step_table_width=step_table[2][1] if step_table else 0,
-        max_new_tokens=min(step.max_new_tokens, _INT32_MAX),
-        max_context=min(step.max_context, _INT32_MAX),
-        max_query_tokens=step.num_query_tokens,
-        max_context_tokens=step.num_context_tokens,
-        max_decode_items=step.num_decode_items,
-        max_merge_items=step.num_merge_items,
-        max_prefill_items=step.num_prefill_items,
+    fields = step._layout.fields
+    step_table = fields.get("block_tables")
+    dims = _native.PaPackDims(  # (in the order of its fields)
+        b,
+        step.block_size,
+        step.table_width,
+        step.partition_size,
+        step.prefill_tile,
+        step._source_rows,
+        n_upd,
+        step_table[2][1] if step_table else 0,
+        min(step.max_new_tokens, _INT32_MAX),
+        min(step.max_context, _INT32_MAX),
+        step.num_query_tokens,
+        step.num_context_tokens,
+        step.num_decode_items,
+        step.num_merge_items,
+        step.num_prefill_items,
     )
-    ws_off, _, ws_shape = step._layout.fields["pack_workspace"]
+    ws_off, _, ws_shape = fields["pack_workspace"]
     clear, clear_bytes = step._merge_state_region()
+    base = step._base
+    stream = _stream(device)
     status = lib.pa_pack(
         table.data_ptr() if table.numel() else None,
         dev + o_rows if pooled and dev else None,
@@ -545,25 +569,25 @@ def _run_pack(step: PackedStep, with_gather: bool = False, updates: Optional[np.
         dev or None,
         dev + o_counts if dev else None,
         dims,
-        step._base + step_table[0] if step_table else None,
-        step.ptr("rows") if pooled else None,
-        step.ptr("cu_seqlens"),
-        step.ptr("cu_context_offsets"),
-        step.ptr("context_lens"),
-        step.ptr("scatter_slots"),
-        step.ptr("position_ids"),
+        base + step_table[0] if step_table else None,
+        base + fields["rows"][0] if pooled else None,
+        base + fields["cu_seqlens"][0],
+        base + fields["cu_context_offsets"][0],
+        base + fields["context_lens"][0],
+        base + fields["scatter_slots"][0],
+        base + fields["position_ids"][0],
         _ptr(gather),
-        step.ptr("decode_items"),
-        step.ptr("merge_items"),
-        step.ptr("prefill_items"),
+        base + fields["decode_items"][0],
+        base + fields["merge_items"][0],
+        base + fields["prefill_items"][0],
         clear,
         clear_bytes,
-        step._base + ws_off,
+        base + ws_off,
         ws_shape[0],
-        _stream(device),
+        stream,
     )
     if staging is not None:
-        staging.done(slot, torch.cuda.current_stream(device))
+        staging.done(slot, device, stream)
     _native.check(status, "pa_pack")
     if fresh and pooled:
         table._pa_pack_generation = _pack_generation(table) + 1
@@ -656,7 +680,7 @@ def pack_step(
     layout.add("merge_items", torch.int32, (int(plan.num_merge_items), 4))
     layout.add("prefill_items", torch.int32, (int(plan.num_prefill_items), 2))
     lib = _native.load_library()
-    layout.add("pack_workspace", torch.uint8, (int(lib.pa_pack_workspace_size(b)),))
+    layout.add("pack_workspace", torch.uint8, (_pack_workspace_size(b),))
     head_shape = None
     ws_bytes = state_bytes = 0
     if head_dim is not None:
@@ -666,7 +690,8 @@ def pack_step(
         ws_dims = _native.PaStepDims(num_seqs=b, num_query_heads=hq, num_kv_heads=int(num_kv_heads),
                                      head_dim=int(head_dim), dtype=dtype_code(dtype or torch.float32))
         ws_bytes = int(lib.pa_decode_workspace_size(ws_dims, int(plan.num_decode_items)))
-        state_bytes = int(lib.pa_decode_merge_state_size(ws_dims, int(plan.num_decode_items)))
+        # (the records follow the partials)
+        state_bytes = ws_bytes - decode_workspace_bytes(int(plan.num_decode_items), hq, int(head_dim))
         layout.add("decode_workspace", torch.uint8, (max(ws_bytes, 1),))
     buffer = torch.empty(layout.nbytes, dtype=torch.uint8, device=device)
     rows_arr = None if rows is None else np.ascontiguousarray(np.asarray(rows, dtype=np.int32).reshape(-1))
@@ -1070,6 +1095,70 @@ def _launch_prefill_append(q, key_cache, value_cache, layer_idx, step, scaling, 
     )
 
 
+def _step_call(step: PackedStep, dims: _native.PaStepDims) -> _native.PaStepCall:
+    """The arguments the layers of ``step`` share."""
+    call = _native.PaStepCall()
+    call.dims = dims
+    call.block_tables = step.ptr("block_tables")
+    call.context_lens = step.ptr("context_lens")
+    call.cu_seqlens = step.ptr("cu_seqlens")
+    call.num_decode_items = step.num_decode_items
+    call.num_merge_items = step.num_merge_items
+    call.num_prefill_items = step.num_prefill_items
+    call.decode_items = step.ptr("decode_items") if step.num_decode_items else None
+    call.merge_items = step.ptr("merge_items") if step.num_merge_items else None
+    call.prefill_items = step.ptr("prefill_items") if step.num_prefill_items else None
+    call.scatter_slots = step.ptr("scatter_slots")
+    call.workspace, call.workspace_bytes = step.workspace_ptr(dims) if step.num_decode_items else (None, 0)
+    call.prefill_tile = step.prefill_tile
+    return call
+
+
+def _attention_step(query, key_cache, value_cache, layer_idx, step, scaling, out, new_key, new_value,
+                    fused_prefill_write) -> Optional[torch.Tensor]:
+    """:func:`attention` with new rows as one library call, or None for what
+    the general path does first (copies of strided rows, an empty step).  The
+    checks and the shared arguments of the last call on ``step`` are kept,
+    keyed by everything they depend on, so a layer after the first costs the
+    key, the output and the call."""
+    key = (query.shape, query.stride(), query.dtype, query.device, key_cache.data_ptr(), value_cache.data_ptr(),
+           key_cache.shape, key_cache.stride(), key_cache.dtype, value_cache.shape, value_cache.stride(),
+           value_cache.dtype, new_key.shape, new_key.stride(), new_key.dtype, new_key.device, new_value.shape,
+           new_value.stride(), new_value.dtype, new_value.device)
+    cached = step.__dict__.get("_layer_call")
+    if cached is None or cached[0] != key:
+        if step.num_prefill_items == 0 and step.num_decode_items == 0:
+            return None
+        if query.stride(-1) != 1 or new_key.stride(-1) != 1 or new_value.stride(-1) != 1:
+            return None
+        q, dims = _checked(query, key_cache, value_cache, step)
+        k, v = _new_rows(new_key, new_value, key_cache, step)
+        call = _step_call(step, dims)
+        # (the step's workspace of other head counts stays alive with the call)
+        cached = (key, ctypes.byref(call), tuple(q.shape), (k.stride(0), k.stride(1), v.stride(0), v.stride(1)),
+                  step._extra_ws)
+        step.__dict__["_layer_call"] = cached
+    _, call_ref, shape, strides, _ = cached
+    if out is None:
+        rows_out = torch.empty(shape, dtype=key_cache.dtype, device=query.device)
+    else:
+        rows_out = _output_for(_query_view(query), key_cache, out)
+    flags = _native.PA_STEP_NO_APPEND if step.__dict__.get("_no_append") else 0
+    if fused_prefill_write is None:
+        fused_prefill_write = key_cache.dtype != torch.float32 and step.num_decode_items == 0
+    if fused_prefill_write:
+        flags |= _native.PA_STEP_PREFILL_WRITE
+    rows = _native.PaNewRows(new_key.data_ptr(), new_value.data_ptr(), *strides)
+    declined = ctypes.c_int32(0)
+    status = _native.load_library().pa_attention_step(
+        call_ref, query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), int(layer_idx),
+        ctypes.byref(rows), float(scaling), rows_out.data_ptr(), flags, ctypes.byref(declined), _stream(query.device))
+    if declined.value:
+        step.__dict__["_no_append"] = True
+    _native.check(status, "pa_attention_step")
+    return rows_out
+
+
 def _fused(status: int, who: str) -> bool:
     """True if a fused-write launch ran, False if it declined the shape."""
     if status == _native.PA_OK:
@@ -1111,10 +1200,15 @@ def attention(
     cheaper per step than the fused writes.  A decode-only step writes its
     rows inside the decode launches.
     """
-    q, dims = _checked(query, key_cache, value_cache, step)
-    out = _output_for(q, key_cache, out)
     if (new_key is None) != (new_value is None):
         raise ValueError("new_key and new_value are given together")
+    if new_key is not None:
+        got = _attention_step(query, key_cache, value_cache, layer_idx, step, scaling, out, new_key, new_value,
+                              fused_prefill_write)
+        if got is not None:
+            return got
+    q, dims = _checked(query, key_cache, value_cache, step)
+    out = _output_for(q, key_cache, out)
     need_prefill = step.num_prefill_items > 0
     need_decode = step.num_decode_items > 0
     if new_key is not None:

@@ -286,3 +286,17 @@ def test_map_host_memory_rejects_unpinned_and_null():
     out = ctypes.c_void_p()
     assert lib.pa_map_host_memory(None, ctypes.byref(out)) == native.PA_ERR_INVALID_ARGUMENT
     assert b"NULL" in lib.pa_last_error_message()
+
+
+def test_attention_step_rejects_null_arguments():
+    native = pkg("_native")
+    lib = native.load_library()
+    call, rows, declined = native.PaStepCall(), native.PaNewRows(), ctypes.c_int32(7)
+    full = [ctypes.byref(call), None, None, None, 0, ctypes.byref(rows), 1.0, None, 0, ctypes.byref(declined), None]
+    for i in (0, 5, 9):
+        args = list(full)
+        args[i] = None
+        assert lib.pa_attention_step(*args) == native.PA_ERR_INVALID_ARGUMENT
+    # rows given without buffers
+    call.dims.num_query_tokens = 1
+    assert lib.pa_attention_step(*full) == native.PA_ERR_INVALID_ARGUMENT and declined.value == 0
