@@ -1095,6 +1095,21 @@ def _launch_prefill_append(q, key_cache, value_cache, layer_idx, step, scaling, 
     )
 
 
+# Most new tokens of a step with decodes that writes its prefill chunks' rows
+# inside the prefill launch: one launch less.  Per layer, apart -> fused: 24
+# decodes and 502 tokens of a 9/3-head model 20.8 -> 19.5 us, 16 and 80 of 32/8
+# heads of 128 25.9 -> 24.8, 64 and 576 137.1 -> 132.9, 16 and 1040 44.7 -> 43.3
+# (42.4 -> 42.7 launched one by one), 128 and 2176 427.0 -> 428.6.
+_MIXED_PREFILL_WRITE_TOKENS = 1024
+
+
+def _writes_in_prefill(key_cache: torch.Tensor, step: PackedStep) -> bool:
+    """Whether the multi-token sequences' new rows are written inside the
+    prefill launch by default (see :func:`attention`)."""
+    return key_cache.dtype != torch.float32 and (
+        step.num_decode_items == 0 or step.num_query_tokens <= _MIXED_PREFILL_WRITE_TOKENS)
+
+
 def _step_call(step: PackedStep, dims: _native.PaStepDims) -> _native.PaStepCall:
     """The arguments the layers of ``step`` share."""
     call = _native.PaStepCall()
@@ -1145,7 +1160,7 @@ def _attention_step(query, key_cache, value_cache, layer_idx, step, scaling, out
         rows_out = _output_for(_query_view(query), key_cache, out)
     flags = _native.PA_STEP_NO_APPEND if step.__dict__.get("_no_append") else 0
     if fused_prefill_write is None:
-        fused_prefill_write = key_cache.dtype != torch.float32 and step.num_decode_items == 0
+        fused_prefill_write = _writes_in_prefill(key_cache, step)
     if fused_prefill_write:
         flags |= _native.PA_STEP_PREFILL_WRITE
     rows = _native.PaNewRows(new_key.data_ptr(), new_value.data_ptr(), *strides)
@@ -1194,10 +1209,9 @@ def attention(
     inside the prefill launch.  By default: on a step of prefill chunks
     alone, for 16-bit caches (fp32 prefills measured 2-4 % slower with the
     write inside than after the cache-write kernel); on a step with decodes
-    too, never -- there the prefill that follows the long decode launch
-    read its chunks' new rows 5-6 us slower than the same rows from the
-    cache, and the cache-write kernel and plain launches measured 4-5 us
-    cheaper per step than the fused writes.  A decode-only step writes its
+    too, up to 1024 new tokens -- on larger ones the prefill read its chunks'
+    new rows more slowly than the same rows from the cache, and the
+    cache-write kernel and plain launches were as fast or faster.  A decode-only step writes its
     rows inside the decode launches.
     """
     if (new_key is None) != (new_value is None):
@@ -1214,7 +1228,7 @@ def attention(
     if new_key is not None:
         k, v = _new_rows(new_key, new_value, key_cache, step)
         if fused_prefill_write is None:
-            fused_prefill_write = key_cache.dtype != torch.float32 and not need_decode
+            fused_prefill_write = _writes_in_prefill(key_cache, step)
         fused = False  # a fused launch wrote rows
         if not step.__dict__.get("_no_append"):
             declined = False
