@@ -1,7 +1,7 @@
 // Paged-attention decode for gfx950 on the vector units: one workgroup per
 // (sequence, context partition of up to 4096 tokens, KV head), split-K merge
-// after.  fp32 caches and 16-bit heads of 80, 96 and 256 run here; 16-bit
-// heads of 64 and 128 run on the matrix cores (decode_mfma.hip).
+// after.  fp32 caches and 16-bit heads of 256 run here; 16-bit heads of 64 to
+// 128 run on the matrix cores (decode_mfma.hip).
 //
 // The workgroup (4 waves) serves the G = H_q / H_kv query heads that share
 // one KV head, so every K/V row of the partition is read from HBM once
@@ -187,7 +187,7 @@ __device__ __forceinline__ float across_groups_max(float x) {
 // SHARED: the workgroup is one of several sub-groups of a KV head's query
 // heads, whose siblings read the same K/V rows (cached loads).
 // DM: the head dim in memory, when smaller than the lane layout's D (heads
-// of 80 and 96 on the layout of 128, in every dtype).  Lanes whose K pieces or V slice lie
+// of 80 and 96 on the layout of 128).  Lanes whose K pieces or V slice lie
 // past DM read the row's first piece or slice instead (always in bounds);
 // their q pieces are zero, so those K pieces add nothing to the scores, and
 // their accumulators are never stored.
@@ -995,12 +995,8 @@ template <bool SHARED, typename Op>
 static hipError_t visit_shape(int dtype, int head_dim, int g, const Op& op) {
   if (dtype == PA_DTYPE_BF16) {
     if (head_dim == 256) return visit_group<bf16_t, 256, SHARED, 256>(g, op);
-    if (head_dim == 96) return visit_group<bf16_t, 128, SHARED, 96>(g, op);
-    if (head_dim == 80) return visit_group<bf16_t, 128, SHARED, 80>(g, op);
   } else if (dtype == PA_DTYPE_F16) {
     if (head_dim == 256) return visit_group<f16_t, 256, SHARED, 256>(g, op);
-    if (head_dim == 96) return visit_group<f16_t, 128, SHARED, 96>(g, op);
-    if (head_dim == 80) return visit_group<f16_t, 128, SHARED, 80>(g, op);
   } else if (dtype == PA_DTYPE_F32) {
     if (head_dim == 128) return visit_group<float, 128, SHARED, 128>(g, op);
     if (head_dim == 64) return visit_group<float, 64, SHARED, 64>(g, op);
@@ -1022,7 +1018,9 @@ static hipError_t visit_decode(int dtype, int head_dim, int group, const Op& op)
 }
 
 int decode_unit_heads(int dtype, int head_dim, int num_kv_heads, int group) {
-  return decode_uses_mfma(dtype, head_dim) && num_kv_heads % 2 == 0 && group >= 1 && group <= 4 ? 2 : 1;
+  return decode_uses_mfma(dtype, head_dim) && head_dim % 64 == 0 && num_kv_heads % 2 == 0 && group >= 1 && group <= 4
+             ? 2
+             : 1;
 }
 
 int decode_sub_groups(int group) {

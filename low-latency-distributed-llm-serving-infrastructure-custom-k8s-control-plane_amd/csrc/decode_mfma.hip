@@ -1,7 +1,7 @@
-// Paged-attention decode of 16-bit caches on the matrix cores: one workgroup
-// per (sequence, context partition, KV head or two adjacent ones), up to 16
-// query heads of a KV head in one pass (larger groups run as sub-groups of at
-// most 16).
+// Paged-attention decode of 16-bit caches on the matrix cores (heads of 64 and
+// 128, and of 80 and 96 on the LDS rows of 128): one workgroup per (sequence,
+// context partition, KV head or two adjacent ones), up to 16 query heads of a
+// KV head in one pass (larger groups run as sub-groups of at most 16).
 //
 // What bounds it is HBM: every K/V byte is read once for all 16 heads, and a
 // 32-token tile costs a wave 16 MFMAs and about 100 vector instructions
@@ -31,6 +31,8 @@
 //                lane's pieces, so the transpose is v_perm_b32 on its own
 //                registers.  The result gives the lane PE * 4 consecutive
 //                dims of head r, whose softmax state it also holds.
+// Heads of 96, 64 sequences of 128-4096 tokens, 32/32: 347 -> 311 us; of 80, 32
+// sequences: 177 -> 148 us; 96/8 heads of 96, 32 sequences: 77 -> 52 us.
 // K as operand loads straight from HBM (64 bytes of 16 rows an instruction,
 // no LDS) took 164 us in the first of those steps; streaming (nontemporal)
 // loads are worth 11-13 % where no sibling reads the rows again.
@@ -88,14 +90,16 @@ __device__ __forceinline__ V row_load(const void* p) {
   return *reinterpret_cast<const V*>(p);
 }
 
-template <typename T, int D, bool SHARED, int HEADS>
+template <typename T, int D, int DM, bool SHARED, int HEADS>
 __global__ __launch_bounds__(kDecodeThreads) __attribute__((amdgpu_waves_per_eu(3))) void
 decode_mfma_kernel(DecodeArgs a) {
   static_assert(sizeof(T) == 2, "16-bit caches");
-  constexpr bool kNt = !SHARED;
+  // (Rows of 160 or 192 bytes share 128-byte lines with the next head's.)
+  constexpr bool kNt = !SHARED && DM == D;
   constexpr int KJ = D / 32;       // MFMAs of a 16-token half's scores
   constexpr int PE = D / 16;       // V elements of a lane's piece, blocks of the output
-  constexpr int kRowBytes = D * 2;
+  constexpr int kRowBytes = D * 2;   // an LDS row
+  constexpr int kMemBytes = DM * 2;  // a cache row
   constexpr int kAccRow = D + 4;   // padded LDS row of one head's accumulators
   using VP = typename VPiece<D>::type;
 
@@ -125,7 +129,7 @@ decode_mfma_kernel(DecodeArgs a) {
   // heads: 208 -> 196 us), but not its heads of 128 (256 sequences, 32/8 heads:
   // 258 us spread over the XCDs, 265 as one gang).
   const int units = hkv / HEADS;
-  const int gang_heads = D == 64 ? units : 1;
+  const int gang_heads = kMemBytes % 256 != 0 ? units : 1;
   const int gang = gang_heads * a.sub_groups;
   const int64_t run = blockIdx.x / (kXcds * gang);
   const int at_run = static_cast<int>(blockIdx.x - run * (kXcds * gang));
@@ -160,18 +164,19 @@ decode_mfma_kernel(DecodeArgs a) {
   // (both scalar loads issued before either is waited for: one round trip)
   asm volatile("" : "+s"(ctx), "+s"(qtok));
   const int n = max(0, min(a.partition, ctx - p0));
-  const int64_t row_bytes = static_cast<int64_t>(hkv) * kRowBytes;
-  const char* kbase = reinterpret_cast<const char*>(a.key_cache) + kvh * kRowBytes;
-  const char* vbase = reinterpret_cast<const char*>(a.value_cache) + kvh * kRowBytes;
+  const int64_t row_bytes = static_cast<int64_t>(hkv) * kMemBytes;
+  const char* kbase = reinterpret_cast<const char*>(a.key_cache) + kvh * kMemBytes;
+  const char* vbase = reinterpret_cast<const char*>(a.value_cache) + kvh * kMemBytes;
 
-  // The query heads (zero past the group).
+  // The query heads (zero past the group and past the head dim).
   u32x4m q[KJ];
 #pragma unroll
   for (int j = 0; j < KJ; ++j) {
     const T* qrow = reinterpret_cast<const T*>(a.query) + qtok * a.q_token_stride +
                     static_cast<int64_t>(h0 + min(r, G - 1)) * a.q_head_stride;
-    const u32x4m x = *reinterpret_cast<const u32x4m*>(qrow + (4 * j + c) * 8);
-    q[j] = r < G ? x : u32x4m{0, 0, 0, 0};
+    const bool in = DM == D || (4 * j + c) * 8 < DM;
+    const u32x4m x = *reinterpret_cast<const u32x4m*>(qrow + (in ? (4 * j + c) * 8 : 0));
+    q[j] = r < G && in ? x : u32x4m{0, 0, 0, 0};
   }
 
   // pa_decode_append: the wave that attends the partition's last tile (which
@@ -179,7 +184,7 @@ decode_mfma_kernel(DecodeArgs a) {
   // head, a lane per 16-byte piece, just before that tile's loads; it loads
   // the pieces here, beside the block ids.  No other wave or workgroup of the
   // launch reads the position (sibling sub-groups write the same bytes).
-  constexpr int kAppendPieces = kRowBytes / 16;
+  constexpr int kAppendPieces = kMemBytes / 16;
   const int ntiles = (n + kMfmaTile - 1) / kMfmaTile;
   const bool append = a.new_key != nullptr && n > 0 && p0 + n == ctx;
   const bool append_wave = append && (ntiles - 1) % kHeadWaves == wave % kHeadWaves;
@@ -224,7 +229,14 @@ decode_mfma_kernel(DecodeArgs a) {
   // first row.
   auto k_row = [&](int i) { return kRowsPerLoad * i + lane / kChunks; };
   auto k_chunk = [&](int i) { return static_cast<uint32_t>(((lane % kChunks) ^ swizzle(k_row(i))) * 16); };
+  // Lanes whose chunk lies past the head dim load nothing: their LDS chunks
+  // stay zero.
+  if constexpr (DM < D) {
+    for (int i = lane; i < kMfmaTile * kChunks; i += kWave) st16(s_k + 16 * i, make_uint4(0, 0, 0, 0));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
   auto load_k_lds = [&](const char* src, int s, int i) {
+    if (DM < D && k_chunk(i) >= kMemBytes) return;
     typedef const __attribute__((address_space(1))) void* global_ptr;
     typedef __attribute__((address_space(3))) void* lds_ptr;
     __builtin_amdgcn_global_load_lds((global_ptr)(src), (lds_ptr)(s_k + (s * kLoads + i) * (kWave * 16)), 16, 0,
@@ -233,7 +245,10 @@ decode_mfma_kernel(DecodeArgs a) {
   uint32_t koff[kLoads];
 #pragma unroll
   for (int i = 0; i < kLoads; ++i) koff[i] = static_cast<uint32_t>(k_row(i) * static_cast<int>(row_bytes)) + k_chunk(i);
-  const uint32_t voff = static_cast<uint32_t>(4 * c * static_cast<int>(row_bytes) + r * (PE * 2));
+  // (Lanes past the head dim read the row's first piece; their output rows
+  // are never stored.)
+  const uint32_t vcol = DM == D || r * PE < DM ? r * (PE * 2) : 0;
+  const uint32_t voff = static_cast<uint32_t>(4 * c * static_cast<int>(row_bytes)) + vcol;
   auto write_new_rows = [&](int tile) {
     if (append_wave && tile == ntiles - 1) {
       if (append_dst != nullptr) st16(append_dst, append_piece);
@@ -281,7 +296,7 @@ decode_mfma_kernel(DecodeArgs a) {
         load_k_lds(kbase + slot_of(t0 + 16 * s + k_row(i)) * row_bytes + k_chunk(i), s, i);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        vt[4 * s + i] = row_load<VP, kNt>(vbase + slot_of(t0 + 16 * s + 4 * c + i) * row_bytes + r * (PE * 2));
+        vt[4 * s + i] = row_load<VP, kNt>(vbase + slot_of(t0 + 16 * s + 4 * c + i) * row_bytes + vcol);
     }
   };
 
@@ -409,13 +424,13 @@ decode_mfma_kernel(DecodeArgs a) {
   const int hq = hkv * a.group;
   const int nparts = (ctx + a.partition - 1) / a.partition;
   const int hu = unit * HEADS * a.group + sg * G;  // first query head of the workgroup
-  float* pacc = a.part_acc + (item * hq + hu) * D;
-  T* out = reinterpret_cast<T*>(a.output) + (qtok * hq + hu) * D;
-  for (int i = tid; i < HEADS * G * D; i += kDecodeThreads) {
-    const int hg = i / D;
+  float* pacc = a.part_acc + (item * hq + hu) * DM;
+  T* out = reinterpret_cast<T*>(a.output) + (qtok * hq + hu) * DM;
+  for (int i = tid; i < HEADS * G * DM; i += kDecodeThreads) {
+    const int hg = i / DM;
     const int w0 = HEADS == 1 ? 0 : hg / G * kHeadWaves;  // the head's first wave
     const int g = HEADS == 1 ? hg : hg % G;
-    const int e = g * kAccRow + (i - hg * D);
+    const int e = g * kAccRow + (i - hg * DM);
     float mx = s_m[w0][g];
 #pragma unroll
     for (int w = 1; w < kHeadWaves; ++w) mx = fmaxf(mx, s_m[w0 + w][g]);
@@ -430,7 +445,7 @@ decode_mfma_kernel(DecodeArgs a) {
       store_scalar<T>(out + i, sum > 0.f ? o / sum : 0.f);
     } else {
       store_device(pacc + i, o);
-      if (i % D == 0) {
+      if (i % DM == 0) {
         float* pml = a.part_ml + (item * hq + hu + hg) * 2;
         store_device(pml, mx);
         store_device(pml + 1, sum);
@@ -438,30 +453,39 @@ decode_mfma_kernel(DecodeArgs a) {
     }
   }
   if (nparts > 1 && n > 0 && a.merge_state != nullptr && seq >= 0 && seq < a.num_seqs)
-    merge_in_launch<T, D, kMergeOutputs>(a, HEADS * G, part, item, ctx, nparts,
+    merge_in_launch<T, DM, kMergeOutputs>(a, HEADS * G, part, item, ctx, nparts,
                                          (static_cast<int64_t>(seq) * units + unit) * a.sub_groups + sg, hu, hq,
-                                         reinterpret_cast<T*>(a.output) + qtok * hq * D);
+                                         reinterpret_cast<T*>(a.output) + qtok * hq * DM);
 }
 
 bool decode_uses_mfma(int dtype, int head_dim) {
-  return (dtype == PA_DTYPE_BF16 || dtype == PA_DTYPE_F16) && (head_dim == 64 || head_dim == 128);
+  return (dtype == PA_DTYPE_BF16 || dtype == PA_DTYPE_F16) &&
+         (head_dim == 64 || head_dim == 80 || head_dim == 96 || head_dim == 128);
 }
 
-template <typename T, int D, typename Op>
+template <typename T, int D, int DM, typename Op>
 static hipError_t visit_mfma_t(bool shared, int heads, const Op& op) {
-  if (heads == 2) return op.template run<T, D, false, 2>();
-  return shared ? op.template run<T, D, true, 1>() : op.template run<T, D, false, 1>();
+  if constexpr (DM == D)
+    if (heads == 2) return op.template run<T, D, DM, false, 2>();
+  return shared ? op.template run<T, D, DM, true, 1>() : op.template run<T, D, DM, false, 1>();
+}
+
+// Heads of 80 and 96 run on the LDS rows of 128.
+template <typename T, typename Op>
+static hipError_t visit_mfma_dim(int head_dim, bool shared, int heads, const Op& op) {
+  switch (head_dim) {
+    case 64: return visit_mfma_t<T, 64, 64>(shared, heads, op);
+    case 80: return visit_mfma_t<T, 128, 80>(shared, heads, op);
+    case 96: return visit_mfma_t<T, 128, 96>(shared, heads, op);
+    case 128: return visit_mfma_t<T, 128, 128>(shared, heads, op);
+    default: return hipErrorNotSupported;
+  }
 }
 
 template <typename Op>
 static hipError_t visit_mfma(int dtype, int head_dim, bool shared, int heads, const Op& op) {
-  if (dtype == PA_DTYPE_BF16) {
-    if (head_dim == 128) return visit_mfma_t<bf16_t, 128>(shared, heads, op);
-    if (head_dim == 64) return visit_mfma_t<bf16_t, 64>(shared, heads, op);
-  } else if (dtype == PA_DTYPE_F16) {
-    if (head_dim == 128) return visit_mfma_t<f16_t, 128>(shared, heads, op);
-    if (head_dim == 64) return visit_mfma_t<f16_t, 64>(shared, heads, op);
-  }
+  if (dtype == PA_DTYPE_BF16) return visit_mfma_dim<bf16_t>(head_dim, shared, heads, op);
+  if (dtype == PA_DTYPE_F16) return visit_mfma_dim<f16_t>(head_dim, shared, heads, op);
   return hipErrorNotSupported;
 }
 
@@ -469,10 +493,10 @@ struct MfmaLaunch {
   const DecodeArgs& a;
   int64_t num_items;
   hipStream_t stream;
-  template <typename T, int D, bool SHARED, int HEADS>
+  template <typename T, int D, int DM, bool SHARED, int HEADS>
   hipError_t run() const {
     const int64_t grid = num_items * (a.num_kv_heads / HEADS) * a.sub_groups;
-    hipLaunchKernelGGL((decode_mfma_kernel<T, D, SHARED, HEADS>), dim3(static_cast<uint32_t>(grid)),
+    hipLaunchKernelGGL((decode_mfma_kernel<T, D, DM, SHARED, HEADS>), dim3(static_cast<uint32_t>(grid)),
                        dim3(kDecodeThreads), 0, stream, a);
     return hipGetLastError();
   }
@@ -480,9 +504,9 @@ struct MfmaLaunch {
 
 struct MfmaOccupancy {
   int* per_cu;
-  template <typename T, int D, bool SHARED, int HEADS>
+  template <typename T, int D, int DM, bool SHARED, int HEADS>
   hipError_t run() const {
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, decode_mfma_kernel<T, D, SHARED, HEADS>,
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, decode_mfma_kernel<T, D, DM, SHARED, HEADS>,
                                                         kDecodeThreads, 0);
   }
 };

@@ -96,6 +96,12 @@ constexpr double kMfmaWorkgroupUs = 0.003;
 constexpr double kMfmaMergeUs = 0.96;
 constexpr double kMfmaMergeUsPerBatch = 0.99;
 constexpr int64_t kMinFullChipMfmaPartition = 1024;
+// Heads of 80 and 96 (whose rows share cache lines with the next head's) keep
+// the rule from 512 tokens on and take at most 256 below it: 64 sequences of
+// 128-4096 tokens, 24/6 heads of 96, 64.9 us at the rule's 512 (76.5 at 4096);
+// 8 of 128-2048, 32/32 heads, 23.1 us at 256 (24.7 at 512, 25.8 at 1024).
+constexpr int64_t kMinFullChipPaddedPartition = 512;
+constexpr int64_t kMaxPaddedPartition = 256;
 
 int64_t choose_partition_mfma(const DecodeContexts& d, const PaPlanParams& p, int dtype, int head_dim,
                               int64_t longest) {
@@ -106,7 +112,8 @@ int64_t choose_partition_mfma(const DecodeContexts& d, const PaPlanParams& p, in
   const int64_t width = p.workgroups_per_item > 0 ? p.workgroups_per_item : hkv;
   const int64_t unit_slots = (p.compute_units > 0 ? p.compute_units : 256) *
                              (p.workgroups_per_cu > 0 ? p.workgroups_per_cu : 3);
-  if (rule >= kMinFullChipMfmaPartition && d.workgroups(rule, width) >= 3 * unit_slots / 2) return rule;
+  const bool padded = head_dim % 64 != 0;
+  if (rule >= (padded ? kMinFullChipPaddedPartition : kMinFullChipMfmaPartition) && d.workgroups(rule, width) >= 3 * unit_slots / 2) return rule;
   const int64_t tokens = d.workgroups(1, 1);
   if (tokens == 0) return rule;
   // Units that one workgroup serves (sub-groups of 8 heads run two to one).
@@ -116,7 +123,7 @@ int64_t choose_partition_mfma(const DecodeContexts& d, const PaPlanParams& p, in
   const double total_us = static_cast<double>(tokens) * 4.0 * head_dim * static_cast<double>(hkv) / kHbmBytesPerUs;
   int64_t best = kMinPartition;
   double best_us = -1.0;
-  for (int64_t part = kMinPartition; part <= kMaxPartition; part *= 2) {
+  for (int64_t part = kMinPartition; part <= (padded ? kMaxPaddedPartition : kMaxPartition); part *= 2) {
     const int64_t wgs = d.workgroups(part, width) / per_wg;
     const double bytes = wg_row * static_cast<double>(part < longest ? part : longest);
     const double read = bytes / kMfmaBytesPerUs > total_us ? bytes / kMfmaBytesPerUs : total_us;

@@ -1,4 +1,4 @@
-"""The matrix-core decode kernel (16-bit heads of 64 and 128) where it can go
+"""The matrix-core decode kernel (16-bit heads of 64 to 128) where it can go
 wrong: contexts at the edges of its 16- and 32-token tiles and of a partition,
 every query-head count it pads to 16, small blocks, missing blocks, and cache
 rows past a context that hold NaN and infinity."""
@@ -74,19 +74,19 @@ def check(heads, kv_heads, dim, dtype, block, partition, contexts=CONTEXTS, hole
 
 @pytest.mark.parametrize("heads,kv_heads", [(1, 1), (3, 3), (9, 3), (10, 2), (7, 1), (16, 2), (9, 1), (22, 2), (16, 1),
                                             (17, 1), (40, 2), (64, 1), (2, 2), (12, 4), (16, 4), (4, 4)])
-@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("dim", [64, 80, 96, 128])
 def test_groups(heads, kv_heads, dim):
     check(heads, kv_heads, dim, torch.bfloat16, 16, 128)
 
 
 @pytest.mark.parametrize("block", [1, 2, 4, 8, 16, 32, 64])
 @pytest.mark.parametrize("holes", [False, True])
-@pytest.mark.parametrize("heads,kv_heads,dim", [(16, 1, 128), (15, 3, 64), (8, 2, 128), (4, 4, 64)])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(16, 1, 128), (15, 3, 64), (8, 2, 128), (4, 4, 64), (6, 3, 96)])
 def test_blocks(block, holes, heads, kv_heads, dim):
     check(heads, kv_heads, dim, torch.float16, block, 96, holes=holes)
 
 
 @pytest.mark.parametrize("partition", [32, 64, 4096])
-@pytest.mark.parametrize("heads,kv_heads,dim", [(16, 1, 128), (10, 2, 64), (8, 2, 128), (6, 6, 64)])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(16, 1, 128), (10, 2, 64), (8, 2, 128), (6, 6, 64), (20, 2, 80)])
 def test_partitions(partition, heads, kv_heads, dim):
     check(heads, kv_heads, dim, torch.bfloat16, 16, partition, contexts=[1, 31, 32, 33, 64, 700, 4095, 4096, 4097])
