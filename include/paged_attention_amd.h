@@ -381,7 +381,9 @@ int32_t pa_prefill_tile(int32_t num_query_heads, int32_t num_kv_heads);
 
 /* Decode workgroups of this shape that one compute unit of the current
  * device holds at once (the HIP occupancy calculator on the kernel pa_decode
- * launches for it), or 0 for a shape without a tuned kernel or on a HIP
+ * launches for it), in the units pa_decode_workgroups_per_item counts (a
+ * workgroup that serves several sub-groups of 8 heads counts as that many),
+ * or 0 for a shape without a tuned kernel or on a HIP
  * error (pa_last_error_message then says which).  With the CU count it gives
  * the resident width a host's split-K partition choice aims to fill.  (No
  * counterpart in the reference.) */
