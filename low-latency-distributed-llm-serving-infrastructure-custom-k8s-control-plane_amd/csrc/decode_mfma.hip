@@ -4,8 +4,8 @@
 // KV head in one pass (larger groups run as sub-groups of at most 16).
 //
 // What bounds it is HBM: every K/V byte is read once for all 16 heads, and a
-// 32-token tile costs a wave 16 MFMAs and about 100 vector instructions
-// whatever the group.  The vector kernel (decode.hip) serves at most 8 heads a
+// 32-token tile costs a wave 24 MFMAs (heads of 128) and about 120 vector
+// instructions whatever the group.  The vector kernel (decode.hip) serves at most 8 heads a
 // pass (groups above 8 read K/V again through L2) at a dot2 per head, token
 // and pair of dims.  Vector kernel -> this one, steps of one layer: 48
 // sequences of 512-8192 tokens, 128/8 heads of 128, fp16, 227 -> 148 us (5.4
@@ -31,6 +31,15 @@
 //                lane's pieces, so the transpose is v_perm_b32 on its own
 //                registers.  The result gives the lane PE * 4 consecutive
 //                dims of head r, whose softmax state it also holds.
+// A probability goes into the product as two terms of the cache type, itself
+// rounded and what the rounding left, so that the result is off by its own
+// rounding alone: rounded once, it was exact only where its token set the
+// running maximum, and the error grew with longer partitions and fewer waves a
+// head.  Off 64 bits in bf16 (2-norm), one term -> two: 16 sequences of
+// 256-1024 tokens, 32/8 heads of 128, 2.1e-3 -> 1.7e-3; 48 of 512-8192, 128/8,
+// fp16, 2.7e-4 -> 2.1e-4.  The 8 MFMAs and 20 vector instructions more a tile
+// hide behind the loads: 16 sequences 117.4 -> 118.1 us for 8 layers, 256 of
+// 32-8192 tokens 258.3 -> 258.6, 64 with 32/32 heads 341.7 -> 341.8.
 // Heads of 96, 64 sequences of 128-4096 tokens, 32/32: 347 -> 311 us; of 80, 32
 // sequences: 177 -> 148 us; 96/8 heads of 96, 32 sequences: 77 -> 52 us.
 // K as operand loads straight from HBM (64 bytes of 16 rows an instruction,
@@ -346,7 +355,7 @@ decode_mfma_kernel(DecodeArgs a) {
       m = m_new;
     }
     const float mc = -m * scale;
-    u32x4m p;
+    u32x4m p, rest;  // the probabilities, and what rounding them left
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -354,7 +363,9 @@ decode_mfma_kernel(DecodeArgs a) {
         const float pa = fast_exp2(fmaf(s[h][2 * i], scale, mc));
         const float pb = fast_exp2(fmaf(s[h][2 * i + 1], scale, mc));
         l += pa + pb;
-        p[2 * h + i] = pack_half2<T>(pa, pb);
+        const uint32_t w = pack_half2<T>(pa, pb);
+        p[2 * h + i] = w;
+        rest[2 * h + i] = pack_half2<T>(pa - half_lo<T>(w), pb - half_hi<T>(w));
       }
 #pragma unroll
     for (int w = 0; w < PE / 2; ++w) {
@@ -364,8 +375,8 @@ decode_mfma_kernel(DecodeArgs a) {
         lo[i] = __builtin_amdgcn_perm(vt[2 * i + 1][w], vt[2 * i][w], 0x05040100u);
         hi[i] = __builtin_amdgcn_perm(vt[2 * i + 1][w], vt[2 * i][w], 0x07060302u);
       }
-      acc[2 * w] = mfma16<T>(lo, p, acc[2 * w]);
-      acc[2 * w + 1] = mfma16<T>(hi, p, acc[2 * w + 1]);
+      acc[2 * w] = mfma16<T>(lo, rest, mfma16<T>(lo, p, acc[2 * w]));
+      acc[2 * w + 1] = mfma16<T>(hi, rest, mfma16<T>(hi, p, acc[2 * w + 1]));
     }
   };
 

@@ -97,6 +97,28 @@ __device__ __forceinline__ uint32_t pack_half2<f16_t>(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2cv));
 }
 
+// The two elements of a packed pair as floats.
+template <typename T>
+__device__ __forceinline__ float half_lo(uint32_t w);
+template <typename T>
+__device__ __forceinline__ float half_hi(uint32_t w);
+template <>
+__device__ __forceinline__ float half_lo<bf16_t>(uint32_t w) {
+  return __uint_as_float(w << 16);
+}
+template <>
+__device__ __forceinline__ float half_hi<bf16_t>(uint32_t w) {
+  return __uint_as_float(w & 0xffff0000u);
+}
+template <>
+__device__ __forceinline__ float half_lo<f16_t>(uint32_t w) {
+  return static_cast<float>(__builtin_bit_cast(f16x2cv, w)[0]);
+}
+template <>
+__device__ __forceinline__ float half_hi<f16_t>(uint32_t w) {
+  return static_cast<float>(__builtin_bit_cast(f16x2cv, w)[1]);
+}
+
 // Dot product of two packed pairs of a 16-bit element type, accumulated in
 // fp32 (v_dot2_f32_bf16 / v_dot2_f32_f16).
 template <typename T>
