@@ -46,6 +46,11 @@ CASES = [
     (2, 3, 3, 132, 300, 0.7),
     (2, 2, 1, 256, 8200, 0.1),
     (390, 2, 1, 256, 70, 0.9),
+    # Groups of 4 and 3 on rows of 256: at 16 waves the kernel's largest LDS.
+    (3, 8, 2, 256, 8200, 0.1),
+    (2, 6, 2, 192, 300, 0.7),
+    (200, 8, 2, 256, 90, 0.8),
+    (200, 6, 2, 252, 4099, 0.05),
     (3, 2, 2, 6, 200, 0.5),  # rows of half pieces: the one-wave kernel
 ]
 
