@@ -55,6 +55,8 @@
 // one of its head's with HEADS 2), the next
 // tile's K and V loads in flight under the current tile's arithmetic, no
 // barrier in the loop.
+#include <type_traits>
+
 #include "decode_common.hpp"
 
 namespace pa {
@@ -97,6 +99,46 @@ template <typename V, bool NT>
 __device__ __forceinline__ V row_load(const void* p) {
   if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
   return *reinterpret_cast<const V*>(p);
+}
+
+// The K operands of a tile from the wave's LDS rows, at[j] the LDS address of
+// piece 4j + c of token r and the second half of the tile HALF bytes further.
+// Waits until at most VM vector memory operations are outstanding, the copies
+// into those rows among the ones that are done: the compiler orders an LDS
+// read after such a copy only where it can tell the two by their alias
+// scopes, and then waits for every load in flight.
+template <int KJ, int HALF, int VM>
+__device__ __forceinline__ void read_k(const uint32_t (&at)[KJ], u32x4m (&k)[2][KJ]) {
+  static_assert(KJ >= 2 && KJ <= 4, "heads of 64 to 128");
+  if constexpr (KJ == 2)
+    asm volatile(
+        "s_waitcnt vmcnt(%7)\n\t"
+        "ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\t"
+        "ds_read_b128 %2, %4 offset:%6\n\tds_read_b128 %3, %5 offset:%6\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(k[0][0]), "=&v"(k[0][1]), "=&v"(k[1][0]), "=&v"(k[1][1])
+        : "v"(at[0]), "v"(at[1]), "n"(HALF), "n"(VM)
+        : "memory");
+  else if constexpr (KJ == 3)
+    asm volatile(
+        "s_waitcnt vmcnt(%10)\n\t"
+        "ds_read_b128 %0, %6\n\tds_read_b128 %1, %7\n\tds_read_b128 %2, %8\n\t"
+        "ds_read_b128 %3, %6 offset:%9\n\tds_read_b128 %4, %7 offset:%9\n\tds_read_b128 %5, %8 offset:%9\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(k[0][0]), "=&v"(k[0][1]), "=&v"(k[0][2]), "=&v"(k[1][0]), "=&v"(k[1][1]), "=&v"(k[1][2])
+        : "v"(at[0]), "v"(at[1]), "v"(at[2]), "n"(HALF), "n"(VM)
+        : "memory");
+  else
+    asm volatile(
+        "s_waitcnt vmcnt(%13)\n\t"
+        "ds_read_b128 %0, %8\n\tds_read_b128 %1, %9\n\tds_read_b128 %2, %10\n\tds_read_b128 %3, %11\n\t"
+        "ds_read_b128 %4, %8 offset:%12\n\tds_read_b128 %5, %9 offset:%12\n\t"
+        "ds_read_b128 %6, %10 offset:%12\n\tds_read_b128 %7, %11 offset:%12\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(k[0][0]), "=&v"(k[0][1]), "=&v"(k[0][2]), "=&v"(k[0][3]), "=&v"(k[1][0]), "=&v"(k[1][1]),
+          "=&v"(k[1][2]), "=&v"(k[1][3])
+        : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "n"(HALF), "n"(VM)
+        : "memory");
 }
 
 template <typename T, int D, int DM, bool SHARED, int HEADS>
@@ -316,17 +358,25 @@ decode_mfma_kernel(DecodeArgs a) {
   for (int b = 0; b < PE; ++b) acc[b] = f32x4m{0.f, 0.f, 0.f, 0.f};
 
   f32x4m s[2];  // scores of tokens 4c .. 4c+3 of each half, head r
-  auto scores = [&]() {
+  // LDS addresses of the lane's K operands in the first half.
+  uint32_t k_at[KJ];
+#pragma unroll
+  for (int j = 0; j < KJ; ++j)
+    k_at[j] = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)s_k)) +
+              r * kRowBytes + 16 * ((4 * j + c) ^ swizzle(r));
+  // VM: the operations issued after the tile's K copies (its V loads).
+  auto scores = [&](auto vm) {
+    u32x4m k[2][KJ];
+    read_k<KJ, 16 * kRowBytes, decltype(vm)::value>(k_at, k);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       s[h] = f32x4m{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < KJ; ++j) {
-        const int at_chunk = (4 * j + c) ^ swizzle(r);
-        s[h] = mfma16<T>(*reinterpret_cast<const u32x4m*>(s_k + (16 * h + r) * kRowBytes + 16 * at_chunk), q[j], s[h]);
-      }
+      for (int j = 0; j < KJ; ++j) s[h] = mfma16<T>(k[h][j], q[j], s[h]);
     }
   };
+  using AllDone = std::integral_constant<int, 0>;
+  using VInFlight = std::integral_constant<int, 8>;
   // Tokens past the end or without a block get no weight, and their V rows
   // (uninitialised or infinite, perhaps) are zeroed.
   auto mask = [&](int tile) {
@@ -386,7 +436,7 @@ decode_mfma_kernel(DecodeArgs a) {
       for (; tile < ntiles; tile += kHeadWaves) {
         write_new_rows(tile);
         load_any(tile);
-        scores();
+        scores(AllDone());
         mask(tile);
         attend();
       }
@@ -402,7 +452,7 @@ decode_mfma_kernel(DecodeArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       for (; tile + kHeadWaves < ntiles; tile += kHeadWaves) {
         locate(tile + kHeadWaves);
-        scores();
+        scores(VInFlight());
         write_new_rows(tile + kHeadWaves);
         __builtin_amdgcn_sched_barrier(0);
         load_k();
@@ -411,7 +461,7 @@ decode_mfma_kernel(DecodeArgs a) {
         load_v();
         __builtin_amdgcn_sched_barrier(0);
       }
-      scores();
+      scores(VInFlight());
       mask(tile);
       attend();
     }
