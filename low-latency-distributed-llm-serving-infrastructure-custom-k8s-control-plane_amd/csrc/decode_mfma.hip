@@ -51,10 +51,18 @@
 // the vector kernel that read them as one row: 256 sequences of 32-8192
 // tokens, 32/8 heads of 128, 268 -> 258 us (6.6 TB/s), 64 sequences, 32/32
 // heads, 343 -> 341; one workgroup per head took 274 and 356.
+// A short context is its workgroup's latency: the prologue has one round trip
+// after the other (item; row, context and token; block ids, query and new rows;
+// K and V), so it divides by multiplication, has one barrier and no load that
+// waits for a block id but K and V.  With divisions, a three-barrier reduction
+// and the new rows loaded after their block id: 138 sequences of 25-49 tokens,
+// 32/8 heads of 128, 10.9 -> 9.4 us, 8/8 10.1 -> 8.6; 131 of 22-88, 32/32 heads
+// of 96, 35.5 -> 30.9.  (Three workgroups per CU at heads of 128, where the
+// vector kernel had four or five for groups of 1: 96 sequences of 55 tokens,
+// 20/20 heads, 960 workgroups, take 14.7 us and took 13.5 there.  At four the
+// registers spill 38.)
 // Each wave runs its own online softmax over every fourth tile (every second
-// one of its head's with HEADS 2), the next
-// tile's K and V loads in flight under the current tile's arithmetic, no
-// barrier in the loop.
+// one of its head's with HEADS 2), no barrier in the loop.
 #include <type_traits>
 
 #include "decode_common.hpp"
@@ -141,13 +149,21 @@ __device__ __forceinline__ void read_k(const uint32_t (&at)[KJ], u32x4m (&k)[2][
         : "memory");
 }
 
+// n / d, with rcp = (2^32 - 1) / d from the host: the product's high half is
+// the quotient or one less.  (A division by a runtime value is a chain of some
+// 30 dependent instructions, and the prologue's stood in front of every load.)
+__device__ __forceinline__ uint32_t quotient(uint32_t n, uint32_t d, uint32_t rcp) {
+  const uint32_t q = __umulhi(n, rcp);
+  return n - q * d >= d ? q + 1 : q;
+}
+
 template <typename T, int D, int DM, bool SHARED, int HEADS>
 __global__ __launch_bounds__(kDecodeThreads) __attribute__((amdgpu_waves_per_eu(3))) void
 decode_mfma_kernel(DecodeArgs a) {
   static_assert(sizeof(T) == 2, "16-bit caches");
   // (Rows of 160 or 192 bytes share 128-byte lines with the next head's.)
   constexpr bool kNt = !SHARED && DM == D;
-  constexpr int KJ = D / 32;       // MFMAs of a 16-token half's scores
+  constexpr int KJ = (DM + 31) / 32;  // MFMAs of a 16-token half's scores
   constexpr int PE = D / 16;       // V elements of a lane's piece, blocks of the output
   constexpr int kRowBytes = D * 2;   // an LDS row
   constexpr int kMemBytes = DM * 2;  // a cache row
@@ -155,6 +171,7 @@ decode_mfma_kernel(DecodeArgs a) {
   using VP = typename VPiece<D>::type;
 
   __shared__ int s_blk[kMaxPartition + 2];
+  __shared__ int s_hole[kDecodeWaves];  // a wave met a missing block
   __shared__ float s_m[kDecodeWaves][kMfmaHeads];
   __shared__ float s_l[kDecodeWaves][kMfmaHeads];
   // Per wave: the K rows of its tile, and after the last tile its
@@ -170,7 +187,8 @@ decode_mfma_kernel(DecodeArgs a) {
   const int c = lane >> 4;
   constexpr int kHeadWaves = kDecodeWaves / HEADS;  // waves per KV head
   const int hkv = a.num_kv_heads;
-  const int G = a.group / a.sub_groups;
+  const uint32_t sub_groups = SHARED ? a.sub_groups : 1;
+  const int G = SHARED ? a.group / a.sub_groups : a.group;
   // Workgroup -> (item, KV head, sub-group).  Ids are dealt to the XCDs
   // round-robin: the members of a gang get ids that are equal modulo the XCD
   // count and close together, gang after gang going to the next XCD (runs of
@@ -179,18 +197,24 @@ decode_mfma_kernel(DecodeArgs a) {
   // heads of 64, whose rows of 128 bytes share HBM bursts (128 sequences, 16/8
   // heads: 208 -> 196 us), but not its heads of 128 (256 sequences, 32/8 heads:
   // 258 us spread over the XCDs, 265 as one gang).
-  const int units = hkv / HEADS;
-  const int gang_heads = kMemBytes % 256 != 0 ? units : 1;
-  const int gang = gang_heads * a.sub_groups;
-  const int64_t run = blockIdx.x / (kXcds * gang);
-  const int at_run = static_cast<int>(blockIdx.x - run * (kXcds * gang));
-  const int width = static_cast<int>(min<int64_t>(kXcds, gridDim.x / gang - run * kXcds));
-  const int member = at_run / width;
-  const int64_t g_id = run * kXcds + (at_run - member * width);
-  const int64_t item = g_id / (units / gang_heads);
-  const int unit = static_cast<int>(g_id - item * (units / gang_heads)) * gang_heads + member / a.sub_groups;
+  const uint32_t units = static_cast<uint32_t>(hkv) / HEADS;
+  constexpr bool kGangUnits = kMemBytes % 256 != 0;
+  uint32_t g_id = blockIdx.x, member = 0;
+  if constexpr (kGangUnits || SHARED) {
+    const uint32_t gang = (kGangUnits ? units : 1) * sub_groups;
+    const uint32_t gangs = static_cast<uint32_t>(a.num_items) * (kGangUnits ? 1 : units);
+    const uint32_t run = quotient(blockIdx.x, kXcds * gang, a.run_rcp);
+    const uint32_t at_run = blockIdx.x - run * (kXcds * gang);
+    const uint32_t width = min(static_cast<uint32_t>(kXcds), gangs - run * kXcds);
+    member = width == kXcds ? at_run / kXcds : at_run / width;
+    g_id = run * kXcds + (at_run - member * width);
+  }
+  const int64_t item = kGangUnits ? g_id : quotient(g_id, units, a.unit_rcp);
+  const int unit = static_cast<int>(!kGangUnits ? g_id - static_cast<uint32_t>(item) * units
+                                    : SHARED    ? member / sub_groups
+                                                : member);
+  const int sg = !SHARED ? 0 : static_cast<int>(kGangUnits ? member - unit * sub_groups : member);
   const int kvh = unit * HEADS + wave / kHeadWaves;
-  const int sg = member % a.sub_groups;
   const int h0 = kvh * a.group + sg * G;  // first query head of the wave
   const int seq = a.items[2 * item];
   const int part = a.items[2 * item + 1];
@@ -219,15 +243,16 @@ decode_mfma_kernel(DecodeArgs a) {
   const char* kbase = reinterpret_cast<const char*>(a.key_cache) + kvh * kMemBytes;
   const char* vbase = reinterpret_cast<const char*>(a.value_cache) + kvh * kMemBytes;
 
-  // The query heads (zero past the group and past the head dim).
+  // The query heads (lanes past the group repeat its last one, and their
+  // results are never stored; zero past the head dim).
   u32x4m q[KJ];
 #pragma unroll
   for (int j = 0; j < KJ; ++j) {
     const T* qrow = reinterpret_cast<const T*>(a.query) + qtok * a.q_token_stride +
                     static_cast<int64_t>(h0 + min(r, G - 1)) * a.q_head_stride;
-    const bool in = DM == D || (4 * j + c) * 8 < DM;
-    const u32x4m x = *reinterpret_cast<const u32x4m*>(qrow + (in ? (4 * j + c) * 8 : 0));
-    q[j] = r < G && in ? x : u32x4m{0, 0, 0, 0};
+    const bool in = DM % 32 == 0 || (4 * j + c) * 8 < DM;
+    q[j] = *reinterpret_cast<const u32x4m*>(qrow + (in ? (4 * j + c) * 8 : 0));
+    if constexpr (DM % 32 != 0) q[j] = in ? q[j] : u32x4m{0, 0, 0, 0};
   }
 
   // pa_decode_append: the wave that attends the partition's last tile (which
@@ -239,21 +264,14 @@ decode_mfma_kernel(DecodeArgs a) {
   const int ntiles = (n + kMfmaTile - 1) / kMfmaTile;
   const bool append = a.new_key != nullptr && n > 0 && p0 + n == ctx;
   const bool append_wave = append && (ntiles - 1) % kHeadWaves == wave % kHeadWaves;
-  char* append_dst = nullptr;
+  const bool append_v = lane >= kAppendPieces;
+  const int append_at = (append_v ? lane - kAppendPieces : lane) * 8;  // element of the piece
   uint4 append_piece = make_uint4(0, 0, 0, 0);
-  if (append_wave && lane < 2 * kAppendPieces) {
-    const int col = (ctx - 1) >> log2_bs;
-    const int b = row_ok && col < a.block_table_stride ? a.block_tables[trow * a.block_table_stride + col] : -1;
-    if (b >= 0 && b < a.total_blocks) {
-      const bool is_v = lane >= kAppendPieces;
-      const int e = (is_v ? lane - kAppendPieces : lane) * 8;
-      append_piece = ld16(reinterpret_cast<const T*>(is_v ? a.new_value : a.new_key) +
-                          qtok * (is_v ? a.new_value_token_stride : a.new_key_token_stride) +
-                          static_cast<int64_t>(kvh) * (is_v ? a.new_value_head_stride : a.new_key_head_stride) + e);
-      const int64_t slot = (static_cast<int64_t>(b) << log2_bs) + ((ctx - 1) & bs_mask);
-      append_dst = const_cast<char*>(is_v ? vbase : kbase) + slot * row_bytes + e * 2;
-    }
-  }
+  if (append_wave && lane < 2 * kAppendPieces)
+    append_piece = ld16(reinterpret_cast<const T*>(append_v ? a.new_value : a.new_key) +
+                        qtok * (append_v ? a.new_value_token_stride : a.new_key_token_stride) +
+                        static_cast<int64_t>(kvh) * (append_v ? a.new_value_head_stride : a.new_key_head_stride) +
+                        append_at);
 
   bool hole = false;  // a block the partition needs is missing
   {
@@ -264,7 +282,12 @@ decode_mfma_kernel(DecodeArgs a) {
     if (tid < nblk) stage(tid, valid_block(b0));
     for (int i = tid + kDecodeThreads; i < nblk; i += kDecodeThreads) stage(i, valid_block(table_entry(i)));
   }
-  hole = __syncthreads_or(hole);
+  hole = __any(hole);
+  if (lane == 0) s_hole[wave] = hole;
+  __syncthreads();
+  hole = false;
+#pragma unroll
+  for (int w = 0; w < kDecodeWaves; ++w) hole |= s_hole[w] != 0;
 
   VP vt[8];  // V of a tile: tokens 4c .. 4c+3 of the first half, then of the second
   // K goes straight into LDS, whole rows per load (in the operand's layout a
@@ -280,10 +303,12 @@ decode_mfma_kernel(DecodeArgs a) {
   // first row.
   auto k_row = [&](int i) { return kRowsPerLoad * i + lane / kChunks; };
   auto k_chunk = [&](int i) { return static_cast<uint32_t>(((lane % kChunks) ^ swizzle(k_row(i))) * 16); };
-  // Lanes whose chunk lies past the head dim load nothing: their LDS chunks
-  // stay zero.
-  if constexpr (DM < D) {
-    for (int i = lane; i < kMfmaTile * kChunks; i += kWave) st16(s_k + 16 * i, make_uint4(0, 0, 0, 0));
+  // Lanes whose chunk lies past the head dim load nothing; the chunks past it
+  // that the scores read (10 and 11 of a head of 80) stay zero.
+  if constexpr (DM % 32 != 0) {
+    static_assert((KJ * 32 - DM) / 8 * kMfmaTile == kWave, "a lane per chunk");
+    const int t = lane % kMfmaTile, chunk = DM / 8 + lane / kMfmaTile;
+    st16(s_k + t * kRowBytes + 16 * (chunk ^ swizzle(t & 15)), make_uint4(0, 0, 0, 0));
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
   auto load_k_lds = [&](const char* src, int s, int i) {
@@ -302,7 +327,10 @@ decode_mfma_kernel(DecodeArgs a) {
   const uint32_t voff = static_cast<uint32_t>(4 * c * static_cast<int>(row_bytes)) + vcol;
   auto write_new_rows = [&](int tile) {
     if (append_wave && tile == ntiles - 1) {
-      if (append_dst != nullptr) st16(append_dst, append_piece);
+      const int b = __builtin_amdgcn_readfirstlane(s_blk[((ctx - 1) >> log2_bs) - first_blk]);
+      const int64_t slot = (static_cast<int64_t>(b) << log2_bs) + ((ctx - 1) & bs_mask);
+      if (b >= 0 && lane < 2 * kAppendPieces)
+        st16(const_cast<char*>(append_v ? vbase : kbase) + slot * row_bytes + append_at * 2, append_piece);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -441,9 +469,16 @@ decode_mfma_kernel(DecodeArgs a) {
         attend();
       }
     } else {
-      // The next tile's K loads go out once the scores have used the current
-      // K, its V loads once the product has used the current V: one register
-      // set, both always in flight.  (The scheduling barriers keep them there.)
+      // The next tile's K copies go out once the scores have used the current
+      // K, its V loads once the product has used the current V: V is in flight
+      // under the scores, the next K under the product.  (The scheduling
+      // barriers keep them there.  With a copy into LDS outstanding the
+      // compiler waits for everything in flight at the first use of a loaded
+      // register, so the empty statements make it wait for the query before
+      // the first copies and for V ahead of the next ones: 1-4 % of a
+      // latency-bound step.)
+#pragma unroll
+      for (int j = 0; j < KJ; ++j) asm volatile("" : "+v"(q[j]));
       write_new_rows(tile);
       locate(tile);
       load_k();
@@ -453,6 +488,8 @@ decode_mfma_kernel(DecodeArgs a) {
       for (; tile + kHeadWaves < ntiles; tile += kHeadWaves) {
         locate(tile + kHeadWaves);
         scores(VInFlight());
+#pragma unroll
+        for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(vt[i]));
         write_new_rows(tile + kHeadWaves);
         __builtin_amdgcn_sched_barrier(0);
         load_k();
@@ -483,14 +520,15 @@ decode_mfma_kernel(DecodeArgs a) {
   __syncthreads();
 
   const int hq = hkv * a.group;
-  const int nparts = (ctx + a.partition - 1) / a.partition;
+  const int nparts = ctx <= a.partition ? 1 : (ctx + a.partition - 1) / a.partition;
   const int hu = unit * HEADS * a.group + sg * G;  // first query head of the workgroup
   float* pacc = a.part_acc + (item * hq + hu) * DM;
   T* out = reinterpret_cast<T*>(a.output) + (qtok * hq + hu) * DM;
   for (int i = tid; i < HEADS * G * DM; i += kDecodeThreads) {
     const int hg = i / DM;
-    const int w0 = HEADS == 1 ? 0 : hg / G * kHeadWaves;  // the head's first wave
-    const int g = HEADS == 1 ? hg : hg % G;
+    const bool second = HEADS == 2 && hg >= G;
+    const int w0 = second ? kHeadWaves : 0;  // the head's first wave
+    const int g = second ? hg - G : hg;
     const int e = g * kAccRow + (i - hg * DM);
     float mx = s_m[w0][g];
 #pragma unroll
@@ -556,9 +594,14 @@ struct MfmaLaunch {
   hipStream_t stream;
   template <typename T, int D, int DM, bool SHARED, int HEADS>
   hipError_t run() const {
-    const int64_t grid = num_items * (a.num_kv_heads / HEADS) * a.sub_groups;
+    const uint32_t units = a.num_kv_heads / HEADS;
+    const int64_t grid = num_items * units * a.sub_groups;
+    const uint32_t gang = (DM * 2 % 256 != 0 ? units : 1) * a.sub_groups;
+    DecodeArgs b = a;
+    b.unit_rcp = 0xffffffffu / units;
+    b.run_rcp = 0xffffffffu / (kXcds * gang);
     hipLaunchKernelGGL((decode_mfma_kernel<T, D, DM, SHARED, HEADS>), dim3(static_cast<uint32_t>(grid)),
-                       dim3(kDecodeThreads), 0, stream, a);
+                       dim3(kDecodeThreads), 0, stream, b);
     return hipGetLastError();
   }
 };

@@ -57,6 +57,10 @@ struct DecodeArgs {
   // kernel combines them.
   int32_t* merge_state;
   int32_t num_seqs;  // sequences the records cover
+  // The matrix-core launch's: (2^32 - 1) / d of the two divisors that map its
+  // workgroups.
+  uint32_t unit_rcp;
+  uint32_t run_rcp;
 };
 
 // Generic one-wave-per-(query token, head) attention: any head_dim <= 256,
