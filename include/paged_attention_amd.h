@@ -263,11 +263,12 @@ int pa_plan_step(const int64_t *start_positions, const int64_t *new_token_counts
 
 /*
  * pa_plan_step for a cache dtype and head dim: where partition_size is 0 and
- * the shape's decode runs on the matrix cores (16-bit heads of 64 and 128), a
- * launch that does not fill the chip at 1024 tokens or more takes the
- * partition of 64 ... 4096 of least modelled time for that kernel, from the
- * step's bytes, its workgroups and the longest sequence's partials.  Any other
- * dtype or head dim: pa_plan_step.
+ * the shape's decode runs on the matrix cores (16-bit heads of 64, 80, 96 and
+ * 128), a launch that does not fill the chip at 2048 tokens or more takes the
+ * partition of 64 ... 4096 (a power of two) of least modelled time for that
+ * kernel, from the step's bytes, its workgroups, the largest of them and the
+ * longest sequence's partials; heads of 80 and 96 have constants of their own.
+ * Any other dtype or head dim: pa_plan_step.
  */
 int pa_plan_step_for(const int64_t *start_positions, const int64_t *new_token_counts,
                      const int64_t *allocated_tokens, int32_t num_seqs,

@@ -79,29 +79,38 @@ int64_t choose_partition(const DecodeContexts& d, const PaPlanParams& p, int64_t
   return best;
 }
 
-// The same for the matrix-core decode kernel (decode_mfma.hip), whose
-// workgroup alone reads 44 GB/s.  A launch that fills the chip at 1024 tokens
-// or more keeps the rule above (its picks are within 2 % of the best).  The
-// model of the others, fitted to 22 graph-replayed steps of 1-64 sequences of
-// 16-16384 tokens (its picks are the fastest power of two on 18 of them and
-// within 6 % on all; the model above lost up to 34 %, 64 sequences of 300-700
-// tokens at 64 instead of 1024: 36.6 against 27.5 us):
-//   read   the step's bytes at 6.45 TB/s, or the largest workgroup's at its own
-//          rate if that takes longer;
-//   launch 0.003 us per workgroup (its prologue and partial stores);
-//   merge  1 us and 1 us more per batch of 8 partials of the longest sequence.
-constexpr double kMfmaBytesPerUs = 43.7e3;
-constexpr double kHbmBytesPerUs = 6.45e6;
-constexpr double kMfmaWorkgroupUs = 0.003;
-constexpr double kMfmaMergeUs = 0.96;
-constexpr double kMfmaMergeUsPerBatch = 0.99;
+// The same for the matrix-core decode kernel (decode_mfma.hip).  A launch that
+// fills the chip at 1024 tokens or more keeps the rule above.  The others take
+// the partition of least modelled time:
+//   read   the largest workgroup's rounds of 128 tokens (64 of each of two KV
+//          heads), a memory round trip each, or the step's bytes at 6.7 TB/s if
+//          that takes longer: plus a share of the former, for while the last
+//          workgroups run alone;
+//   launch a time per workgroup (its prologue and partial stores);
+//   merge  a constant and a time per batch of 8 partials of the longest sequence.
+// Constants per head dim, fitted to 928 steps of 1-160 sequences of 4-65536
+// tokens, 27 head shapes, from a HIP graph over cold layers, where the picks take
+// 1.2 % longer than the best power of two on average and 20 % at most (the model
+// above: 13 % and 104 %).  Two failures of a model of one constant rate a
+// workgroup and no share of the last ones: 49 sequences of 748-1648 tokens, 8/8
+// heads of 64, at 2048, 30.4 us (26.7 at 256); 21 of 7331-15987, 8/8 heads of 128,
+// at 4096, 175 us (165 at 1024).
+struct MfmaModel {
+  double round_us;
+  double tail;
+  double workgroup_us;
+  double merge_us;
+  double merge_us_per_batch;
+};
+constexpr double kHbmBytesPerUs = 6.7e6;
+constexpr int64_t kMfmaRoundTokens = 128;
 constexpr int64_t kMinFullChipMfmaPartition = 1024;
-// Heads of 80 and 96 (whose rows share cache lines with the next head's) keep
-// the rule from 512 tokens on and take at most 256 below it: 64 sequences of
-// 128-4096 tokens, 24/6 heads of 96, 64.9 us at the rule's 512 (76.5 at 4096);
-// 8 of 128-2048, 32/32 heads, 23.1 us at 256 (24.7 at 512, 25.8 at 1024).
-constexpr int64_t kMinFullChipPaddedPartition = 512;
-constexpr int64_t kMaxPaddedPartition = 256;
+constexpr MfmaModel kMfmaModel128 = {1.45, 0.02, 0.00027, 1.9, 1.4};
+constexpr MfmaModel kMfmaModel64 = {1.19, 0.26, 0.0007, 0.63, 2.0};
+// Heads of 80 and 96, whose rows share cache lines with the next head's: two
+// sequences of 20142-27521 tokens, 32/8 heads of 96, 35.2 us at its 2048 (40.4
+// at 1024, 47.4 at 256); 15 of 990-2801, 12/12, 30.3 at its 512 (35.4 at 4096).
+constexpr MfmaModel kMfmaModelPadded = {1.68, 0.3, 0.00019, 2.2, 1.9};
 
 int64_t choose_partition_mfma(const DecodeContexts& d, const PaPlanParams& p, int dtype, int head_dim,
                               int64_t longest) {
@@ -112,25 +121,25 @@ int64_t choose_partition_mfma(const DecodeContexts& d, const PaPlanParams& p, in
   const int64_t width = p.workgroups_per_item > 0 ? p.workgroups_per_item : hkv;
   const int64_t unit_slots = (p.compute_units > 0 ? p.compute_units : 256) *
                              (p.workgroups_per_cu > 0 ? p.workgroups_per_cu : 3);
-  const bool padded = head_dim % 64 != 0;
-  if (rule >= (padded ? kMinFullChipPaddedPartition : kMinFullChipMfmaPartition) && d.workgroups(rule, width) >= 3 * unit_slots / 2) return rule;
+  const MfmaModel& model = head_dim == 128 ? kMfmaModel128 : head_dim == 64 ? kMfmaModel64 : kMfmaModelPadded;
+  if (rule >= kMinFullChipMfmaPartition && d.workgroups(rule, width) >= 3 * unit_slots / 2) return rule;
   const int64_t tokens = d.workgroups(1, 1);
   if (tokens == 0) return rule;
   // Units that one workgroup serves (sub-groups of 8 heads run two to one).
   const int64_t per_wg = pa::decode_sub_groups(group) / pa::decode_workgroups_per_head(dtype, head_dim, group);
   const int heads = pa::decode_unit_heads(dtype, head_dim, static_cast<int>(hkv), group);
-  const double wg_row = 4.0 * head_dim * heads;  // K and V bytes of a token a workgroup reads
   const double total_us = static_cast<double>(tokens) * 4.0 * head_dim * static_cast<double>(hkv) / kHbmBytesPerUs;
   int64_t best = kMinPartition;
   double best_us = -1.0;
-  for (int64_t part = kMinPartition; part <= (padded ? kMaxPaddedPartition : kMaxPartition); part *= 2) {
+  for (int64_t part = kMinPartition; part <= kMaxPartition; part *= 2) {
     const int64_t wgs = d.workgroups(part, width) / per_wg;
-    const double bytes = wg_row * static_cast<double>(part < longest ? part : longest);
-    const double read = bytes / kMfmaBytesPerUs > total_us ? bytes / kMfmaBytesPerUs : total_us;
+    const int64_t rounds = ceil_div((part < longest ? part : longest) * heads, kMfmaRoundTokens);
+    const double own_us = model.round_us * static_cast<double>(rounds);
+    const double read = own_us > total_us + model.tail * own_us ? own_us : total_us + model.tail * own_us;
     const int64_t parts = ceil_div(longest, part);
     const double merge =
-        parts > 1 ? kMfmaMergeUs + kMfmaMergeUsPerBatch * static_cast<double>(ceil_div(parts, kMergeBatch)) : 0.0;
-    const double us = read + kMfmaWorkgroupUs * static_cast<double>(wgs) + merge;
+        parts > 1 ? model.merge_us + model.merge_us_per_batch * static_cast<double>(ceil_div(parts, kMergeBatch)) : 0.0;
+    const double us = read + model.workgroup_us * static_cast<double>(wgs) + merge;
     if (best_us < 0.0 || us < best_us * (1.0 - 1e-9)) {
       best = part;
       best_us = us;
