@@ -235,6 +235,7 @@ class PackedStep:
         self._head_shape = head_shape  # (H_q, D) the workspace was sized for, or None
         self._gather = None
         self._extra_ws = None
+        self._prefill_context = None
         self._generation = 0  # the pool's pack count when this step was packed
         self._merge_state_bytes = 0  # merge records at the end of the decode workspace
 
@@ -295,6 +296,16 @@ class PackedStep:
         """int64 [B] (host) new tokens of every sequence."""
         return self._inputs[1]
 
+    @property
+    def longest_prefill_context(self) -> int:
+        """Longest context after the step of a sequence with several new
+        tokens (0 without one)."""
+        if self._prefill_context is None:
+            starts, counts = self._inputs[0], self._inputs[1]
+            multi = counts > 1
+            self._prefill_context = int((starts + counts)[multi].max()) if multi.any() else 0
+        return self._prefill_context
+
     def repack(self, start_positions=None, new_token_counts=None) -> None:
         """Rerun the packing kernels in place with new positions / counts of
         the same sequences (what a step captured in a graph re-reads): every
@@ -310,6 +321,7 @@ class PackedStep:
         if self.table_width and plan.max_blocks > self.table_width:
             raise ValueError("repack: a context grew past the step's block table")
         self._inputs = (starts, counts, self._inputs[2])
+        self._prefill_context = None
         self.num_context_tokens = int(plan.num_context_tokens)
         self.max_context = int(plan.max_context)
         self._gather = None
@@ -1095,19 +1107,26 @@ def _launch_prefill_append(q, key_cache, value_cache, layer_idx, step, scaling, 
     )
 
 
-# Most new tokens of a step with decodes that writes its prefill chunks' rows
-# inside the prefill launch: one launch less.  Per layer, apart -> fused: 24
-# decodes and 502 tokens of a 9/3-head model 20.8 -> 19.5 us, 16 and 80 of 32/8
-# heads of 128 25.9 -> 24.8, 64 and 576 137.1 -> 132.9, 16 and 1040 44.7 -> 43.3
-# (42.4 -> 42.7 launched one by one), 128 and 2176 427.0 -> 428.6.
+# A step with decodes writes its prefill chunks' rows inside the prefill launch,
+# one launch less, up to this many new tokens and this long a prefill context.
+# Per layer, apart -> fused, beside 4-24 decodes: 4 prompts of 250 tokens, 9/3
+# heads of 64 20.0 -> 18.9 us, 32/8 of 128 27.1 -> 26.5, 64/8 32.4 -> 32.0; 24
+# decodes and 502 tokens, 9/3, 20.8 -> 19.5.  Longer contexts read the chunk's
+# rows for longer from the new rows, which costs more than the launch: 900 tokens
+# at 2000, 32/8, 64.4 -> 66.5; 512 at 8192, 138 -> 152; 128 decodes and 2176
+# tokens 427.0 -> 428.6.  (At 256 tokens groups above 4 of 128 lose 1-2 %, at 512
+# all of 128 do.)
 _MIXED_PREFILL_WRITE_TOKENS = 1024
+_MIXED_PREFILL_WRITE_CONTEXT = 256
 
 
 def _writes_in_prefill(key_cache: torch.Tensor, step: PackedStep) -> bool:
     """Whether the multi-token sequences' new rows are written inside the
     prefill launch by default (see :func:`attention`)."""
-    return key_cache.dtype != torch.float32 and (
-        step.num_decode_items == 0 or step.num_query_tokens <= _MIXED_PREFILL_WRITE_TOKENS)
+    if key_cache.dtype == torch.float32 or step.num_prefill_items == 0:
+        return False
+    return step.num_decode_items == 0 or (step.num_query_tokens <= _MIXED_PREFILL_WRITE_TOKENS and
+                                          step.longest_prefill_context <= _MIXED_PREFILL_WRITE_CONTEXT)
 
 
 def _step_call(step: PackedStep, dims: _native.PaStepDims) -> _native.PaStepCall:
@@ -1209,10 +1228,10 @@ def attention(
     inside the prefill launch.  By default: on a step of prefill chunks
     alone, for 16-bit caches (fp32 prefills measured 2-4 % slower with the
     write inside than after the cache-write kernel); on a step with decodes
-    too, up to 1024 new tokens -- on larger ones the prefill read its chunks'
-    new rows more slowly than the same rows from the cache, and the
-    cache-write kernel and plain launches were as fast or faster.  A decode-only step writes its
-    rows inside the decode launches.
+    too, up to 1024 new tokens and prefill contexts of 256 -- on longer ones the
+    prefill reads its chunks' new rows more slowly than the same rows from the
+    cache, and the cache-write kernel and plain launches are faster.  A
+    decode-only step writes its rows inside the decode launches.
     """
     if (new_key is None) != (new_value is None):
         raise ValueError("new_key and new_value are given together")
