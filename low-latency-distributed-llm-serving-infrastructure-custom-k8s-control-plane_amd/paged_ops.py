@@ -302,8 +302,7 @@ class PackedStep:
         tokens (0 without one)."""
         if self._prefill_context is None:
             starts, counts = self._inputs[0], self._inputs[1]
-            multi = counts > 1
-            self._prefill_context = int((starts + counts)[multi].max()) if multi.any() else 0
+            self._prefill_context = int(np.maximum.reduce((starts + counts) * (counts > 1), initial=0))
         return self._prefill_context
 
     def repack(self, start_positions=None, new_token_counts=None) -> None:
