@@ -235,7 +235,6 @@ class PackedStep:
         self._head_shape = head_shape  # (H_q, D) the workspace was sized for, or None
         self._gather = None
         self._extra_ws = None
-        self._prefill_context = None
         self._generation = 0  # the pool's pack count when this step was packed
         self._merge_state_bytes = 0  # merge records at the end of the decode workspace
 
@@ -296,15 +295,6 @@ class PackedStep:
         """int64 [B] (host) new tokens of every sequence."""
         return self._inputs[1]
 
-    @property
-    def longest_prefill_context(self) -> int:
-        """Longest context after the step of a sequence with several new
-        tokens (0 without one)."""
-        if self._prefill_context is None:
-            starts, counts = self._inputs[0], self._inputs[1]
-            self._prefill_context = int(np.maximum.reduce((starts + counts) * (counts > 1), initial=0))
-        return self._prefill_context
-
     def repack(self, start_positions=None, new_token_counts=None) -> None:
         """Rerun the packing kernels in place with new positions / counts of
         the same sequences (what a step captured in a graph re-reads): every
@@ -320,7 +310,7 @@ class PackedStep:
         if self.table_width and plan.max_blocks > self.table_width:
             raise ValueError("repack: a context grew past the step's block table")
         self._inputs = (starts, counts, self._inputs[2])
-        self._prefill_context = None
+        self.__dict__.pop("_layer_call", None)  # (its default for the prefill write)
         self.num_context_tokens = int(plan.num_context_tokens)
         self.max_context = int(plan.max_context)
         self._gather = None
@@ -1056,56 +1046,6 @@ def _new_rows(new_key: torch.Tensor, new_value: torch.Tensor, key_cache: torch.T
     return new_key, new_value
 
 
-def _launch_decode_append(q, key_cache, value_cache, layer_idx, step, scaling, out, dims, k, v) -> int:
-    """pa_decode_append; returns its status (PA_ERR_UNSUPPORTED: not fused)."""
-    ws_ptr, ws_bytes = step.workspace_ptr(dims)
-    rows = _native.PaNewRows(k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), v.stride(0), v.stride(1))
-    lib = _native.load_library()
-    return lib.pa_decode_append(
-        q.data_ptr(),
-        key_cache.data_ptr(),
-        value_cache.data_ptr(),
-        int(layer_idx),
-        dims,
-        rows,
-        step.ptr("block_tables"),
-        step.ptr("context_lens"),
-        step.ptr("cu_seqlens"),
-        step.ptr("decode_items"),
-        step.num_decode_items,
-        step.ptr("merge_items") if step.num_merge_items else None,
-        step.num_merge_items,
-        float(scaling),
-        out.data_ptr(),
-        ws_ptr,
-        ws_bytes,
-        _stream(q.device),
-    )
-
-
-def _launch_prefill_append(q, key_cache, value_cache, layer_idx, step, scaling, out, dims, k, v) -> int:
-    """pa_prefill_append; returns its status (PA_ERR_UNSUPPORTED: not fused)."""
-    rows = _native.PaNewRows(k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), v.stride(0), v.stride(1))
-    lib = _native.load_library()
-    return lib.pa_prefill_append(
-        q.data_ptr(),
-        key_cache.data_ptr(),
-        value_cache.data_ptr(),
-        int(layer_idx),
-        dims,
-        rows,
-        step.ptr("block_tables"),
-        step.ptr("context_lens"),
-        step.ptr("cu_seqlens"),
-        step.ptr("prefill_items"),
-        step.num_prefill_items,
-        step.prefill_tile,
-        float(scaling),
-        out.data_ptr(),
-        _stream(q.device),
-    )
-
-
 # A step with decodes writes its prefill chunks' rows inside the prefill launch,
 # one launch less, up to this many new tokens and this long a prefill context.
 # Per layer, apart -> fused, beside 4-24 decodes: 4 prompts of 250 tokens, 9/3
@@ -1124,8 +1064,17 @@ def _writes_in_prefill(key_cache: torch.Tensor, step: PackedStep) -> bool:
     prefill launch by default (see :func:`attention`)."""
     if key_cache.dtype == torch.float32 or step.num_prefill_items == 0:
         return False
-    return step.num_decode_items == 0 or (step.num_query_tokens <= _MIXED_PREFILL_WRITE_TOKENS and
-                                          step.longest_prefill_context <= _MIXED_PREFILL_WRITE_CONTEXT)
+    if step.num_decode_items == 0:
+        return True
+    if step.num_query_tokens > _MIXED_PREFILL_WRITE_TOKENS or step.max_new_tokens > _MIXED_PREFILL_WRITE_CONTEXT:
+        return False
+    starts, counts, _ = step._inputs
+    if step.num_seqs > 64:
+        return bool(np.maximum.reduce((starts + counts) * (counts > 1)) <= _MIXED_PREFILL_WRITE_CONTEXT)
+    for start, count in zip(starts.tolist(), counts.tolist()):
+        if count > 1 and start + count > _MIXED_PREFILL_WRITE_CONTEXT:
+            return False
+    return True
 
 
 def _step_call(step: PackedStep, dims: _native.PaStepDims) -> _native.PaStepCall:
@@ -1148,38 +1097,35 @@ def _step_call(step: PackedStep, dims: _native.PaStepDims) -> _native.PaStepCall
 
 
 def _attention_step(query, key_cache, value_cache, layer_idx, step, scaling, out, new_key, new_value,
-                    fused_prefill_write) -> Optional[torch.Tensor]:
-    """:func:`attention` with new rows as one library call, or None for what
-    the general path does first (copies of strided rows, an empty step).  The
-    checks and the shared arguments of the last call on ``step`` are kept,
-    keyed by everything they depend on, so a layer after the first costs the
-    key, the output and the call."""
-    key = (query.shape, query.stride(), query.dtype, query.device, key_cache.data_ptr(), value_cache.data_ptr(),
-           key_cache.shape, key_cache.stride(), key_cache.dtype, value_cache.shape, value_cache.stride(),
-           value_cache.dtype, new_key.shape, new_key.stride(), new_key.dtype, new_key.device, new_value.shape,
-           new_value.stride(), new_value.dtype, new_value.device)
+                    fused_prefill_write) -> torch.Tensor:
+    """:func:`attention` with new rows as one library call, of a step with work
+    items.  The checks and the shared arguments of the last call on ``step``
+    are kept, keyed by everything they depend on, so a layer after the first
+    costs the key, the output and the call.  Rows without unit stride along D
+    are copied first."""
+    qs, ks, vs = query.stride(), new_key.stride(), new_value.stride()
+    if not (qs and ks and vs) or qs[-1] != 1 or ks[-1] != 1 or vs[-1] != 1:
+        query, new_key, new_value = _query_view(query), new_key.contiguous(), new_value.contiguous()
+        qs, ks, vs = query.stride(), new_key.stride(), new_value.stride()
+    key = (query.shape, qs, query.dtype, query.device, key_cache.data_ptr(), value_cache.data_ptr(), key_cache.shape,
+           key_cache.stride(), key_cache.dtype, value_cache.shape, value_cache.stride(), value_cache.dtype,
+           new_key.shape, ks, new_key.dtype, new_key.device, new_value.shape, vs, new_value.dtype, new_value.device)
     cached = step.__dict__.get("_layer_call")
     if cached is None or cached[0] != key:
-        if step.num_prefill_items == 0 and step.num_decode_items == 0:
-            return None
-        if query.stride(-1) != 1 or new_key.stride(-1) != 1 or new_value.stride(-1) != 1:
-            return None
         q, dims = _checked(query, key_cache, value_cache, step)
         k, v = _new_rows(new_key, new_value, key_cache, step)
         call = _step_call(step, dims)
         # (the step's workspace of other head counts stays alive with the call)
         cached = (key, ctypes.byref(call), tuple(q.shape), (k.stride(0), k.stride(1), v.stride(0), v.stride(1)),
-                  step._extra_ws)
+                  _writes_in_prefill(key_cache, step), step._extra_ws)
         step.__dict__["_layer_call"] = cached
-    _, call_ref, shape, strides, _ = cached
+    _, call_ref, shape, strides, write_in_prefill, _ = cached
     if out is None:
         rows_out = torch.empty(shape, dtype=key_cache.dtype, device=query.device)
     else:
         rows_out = _output_for(_query_view(query), key_cache, out)
     flags = _native.PA_STEP_NO_APPEND if step.__dict__.get("_no_append") else 0
-    if fused_prefill_write is None:
-        fused_prefill_write = _writes_in_prefill(key_cache, step)
-    if fused_prefill_write:
+    if write_in_prefill if fused_prefill_write is None else fused_prefill_write:
         flags |= _native.PA_STEP_PREFILL_WRITE
     rows = _native.PaNewRows(new_key.data_ptr(), new_value.data_ptr(), *strides)
     declined = ctypes.c_int32(0)
@@ -1190,15 +1136,6 @@ def _attention_step(query, key_cache, value_cache, layer_idx, step, scaling, out
         step.__dict__["_no_append"] = True
     _native.check(status, "pa_attention_step")
     return rows_out
-
-
-def _fused(status: int, who: str) -> bool:
-    """True if a fused-write launch ran, False if it declined the shape."""
-    if status == _native.PA_OK:
-        return True
-    if status != _native.PA_ERR_UNSUPPORTED:
-        _native.check(status, who)
-    return False
 
 
 def attention(
@@ -1234,37 +1171,16 @@ def attention(
     """
     if (new_key is None) != (new_value is None):
         raise ValueError("new_key and new_value are given together")
-    if new_key is not None:
-        got = _attention_step(query, key_cache, value_cache, layer_idx, step, scaling, out, new_key, new_value,
-                              fused_prefill_write)
-        if got is not None:
-            return got
-    q, dims = _checked(query, key_cache, value_cache, step)
-    out = _output_for(q, key_cache, out)
     need_prefill = step.num_prefill_items > 0
     need_decode = step.num_decode_items > 0
+    if new_key is not None and (need_prefill or need_decode):
+        return _attention_step(query, key_cache, value_cache, layer_idx, step, scaling, out, new_key, new_value,
+                               fused_prefill_write)
+    q, dims = _checked(query, key_cache, value_cache, step)
+    out = _output_for(q, key_cache, out)
     if new_key is not None:
         k, v = _new_rows(new_key, new_value, key_cache, step)
-        if fused_prefill_write is None:
-            fused_prefill_write = _writes_in_prefill(key_cache, step)
-        fused = False  # a fused launch wrote rows
-        if not step.__dict__.get("_no_append"):
-            declined = False
-            if need_prefill and fused_prefill_write:
-                if _fused(_launch_prefill_append(q, key_cache, value_cache, layer_idx, step, scaling, out, dims,
-                                                 k, v), "pa_prefill_append"):
-                    need_prefill, fused = False, True
-                else:
-                    declined = True
-            if need_decode and not need_prefill:
-                if _fused(_launch_decode_append(q, key_cache, value_cache, layer_idx, step, scaling, out, dims,
-                                                k, v), "pa_decode_append"):
-                    need_decode, fused = False, True
-                else:
-                    declined = True
-            if declined:
-                step.__dict__["_no_append"] = True
-        if (need_prefill or need_decode or not fused) and step.num_query_tokens > 0:
+        if step.num_query_tokens > 0:
             reshape_and_cache(k, v, key_cache, value_cache, step.scatter_slots, layer_idx)
     if need_prefill:
         _launch_prefill(q, key_cache, value_cache, layer_idx, step, scaling, out, dims)

@@ -823,6 +823,38 @@ def test_attention_with_new_rows_on_a_mixed_step(device, fused_prefill_write):
     assert torch.equal(_bits(got), _bits(want))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("starts,counts", [([700, 5, 63], [1, 1, 1]), ([0, 300], [90, 40]),
+                                           ([0, 300, 57], [90, 40, 1]), ([], [])])
+@pytest.mark.parametrize("four_dims", [False, True])
+def test_attention_takes_new_rows_of_any_stride(device, dtype, starts, counts, four_dims):
+    """Query and new rows whose elements along D are not adjacent, on steps of
+    decodes, of prefill chunks, of both and of nothing: the bytes and bits of
+    the same rows laid out contiguously, over two layers."""
+    base = wl.prefill_chunks("strided", starts or [3], counts or [1], dtype, 16, 4, 64)
+    w = wl.StepWorkload("strided", 16, 4, 64, 16, dtype, 1.0, base.start_positions, base.new_token_counts,
+                        base.block_lists, base.total_blocks, num_layers=2)
+    t = wl.make_tensors(w, device, seed=8)
+    if starts:
+        step = pack_workload(w, device)
+        query, keys, values = t.query, t.new_keys, t.new_values
+    else:
+        step = ops.pack_step(torch.zeros((0, 4), dtype=torch.int32, device=device), [], [], 16, num_kv_heads=4,
+                             num_query_heads=16, head_dim=64, dtype=dtype)
+        query, keys, values = t.query[:, :, :0], t.new_keys[:0], t.new_values[:0]
+    q3 = query[0].transpose(0, 1)
+    strided = lambda x: torch.stack([x, x], dim=-1)[..., 0]
+    q = strided(query) if four_dims else strided(q3)
+    assert not starts or (q.stride(-1) == 2 and strided(keys).stride(-1) == 2)
+    kc, vc = t.key_cache.clone(), t.value_cache.clone()
+    for layer in (0, 1):
+        want = ops.attention(q3.contiguous(), t.key_cache, t.value_cache, layer, step, 0.125,
+                             new_key=keys.contiguous(), new_value=values.contiguous())
+        got = ops.attention(q, kc, vc, layer, step, 0.125, new_key=strided(keys), new_value=strided(values))
+        assert got.shape == want.shape and torch.equal(_bits(got), _bits(want))
+    assert torch.equal(_bits(kc), _bits(t.key_cache)) and torch.equal(_bits(vc), _bits(t.value_cache))
+
+
 @pytest.mark.parametrize("hq,hkv,d,dtype,bs,fused", [
     (32, 8, 128, torch.bfloat16, 16, True), (16, 16, 128, torch.float16, 32, True),
     (64, 4, 128, torch.bfloat16, 16, True), (16, 2, 96, torch.bfloat16, 16, True),

@@ -562,6 +562,8 @@ def test_partition_of_the_matrix_core_decode(starts, heads, head_dim, want):
     (torch.bfloat16, [57, 9000], [200, 1], False),
     (torch.bfloat16, [8192, 9000], [512, 1], False),       # a chunk of a long prompt
     (torch.bfloat16, [0] * 6 + [9], [200] * 6 + [1], False),   # 1201 tokens
+    (torch.bfloat16, [0, 250] + [900] * 70, [230, 6] + [1] * 70, True),
+    (torch.bfloat16, [0, 250] + [900] * 70, [230, 7] + [1] * 70, False),
     (torch.bfloat16, [8192, 0], [512, 700], True),         # chunks alone
     (torch.bfloat16, [8192], [1], False),                  # nothing to prefill
     (torch.float32, [0, 500], [230, 1], False),
@@ -569,6 +571,6 @@ def test_partition_of_the_matrix_core_decode(starts, heads, head_dim, want):
 def test_which_steps_write_prefill_rows_in_the_prefill_launch(dtype, starts, counts, inside):
     step = ops.PackedStep.__new__(ops.PackedStep)
     step.__dict__.update(_inputs=(np.asarray(starts, dtype=np.int64), np.asarray(counts, dtype=np.int64), None),
-                         _prefill_context=None, num_query_tokens=sum(counts),
+                         num_query_tokens=sum(counts), num_seqs=len(counts), max_new_tokens=max(counts),
                          num_decode_items=sum(c == 1 for c in counts), num_prefill_items=sum(c > 1 for c in counts))
     assert ops._writes_in_prefill(torch.empty(0, dtype=dtype), step) is inside
