@@ -590,7 +590,6 @@ int decode_phases(const char* who, bool use_scratch, int32_t phases, const void*
     a.scale_log2e = scaling * pa::kLog2e;
     a.group = group;
     a.sub_groups = pa::decode_workgroups_per_head(dims.dtype, dims.head_dim, group);
-    a.head_dim = dims.head_dim;
     // A record's fields hold counts and items below 65535.
     a.merge_state = num_decode_items < 65535 ? merge_state : nullptr;
     a.num_seqs = dims.num_seqs;

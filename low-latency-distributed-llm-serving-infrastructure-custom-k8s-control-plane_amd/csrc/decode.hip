@@ -19,14 +19,14 @@
 //                 contiguously); a wave covers 64 / kL tokens per load.
 //                 Dots with the G query slices use v_dot2_f32_bf16 /
 //                 v_dot2_f32_f16 (16-bit types) and a DPP butterfly sums
-//                 each group; groups of more than half a row group use a
-//                 reduce-scatter instead, after which each lane holds one
-//                 head's scores (qk_softmax_rs).
-//  V (PV layout)  one wave load covers whole V rows (one 256-byte row for
-//                 bf16 D=128, 4 bytes per lane), so the row address of a
-//                 load is wave-uniform and is formed in scalar registers
-//                 from the block id fetched with v_readlane.  Every lane
-//                 owns a fixed slice of the head dimension for all G heads.
+//                 each group; groups of more than 4 on fp32 heads of 64 (row
+//                 groups of 8 lanes) use a reduce-scatter instead, after
+//                 which each lane holds one head's scores (qk_softmax_rs).
+//  V (PV layout)  one wave load covers one V row (4 bytes per lane of 256-byte
+//                 rows, 8 of 512), so the row address of a load is
+//                 wave-uniform and is formed in scalar registers from the
+//                 block id fetched with v_readlane.  Every lane owns a fixed
+//                 slice of the head dimension for all G heads.
 //  softmax        per tile: wave-wide max per head (DPP + shuffles), rescale
 //                 of the running sum / accumulator only when the max moved,
 //                 p = exp2(s - max) staged in LDS.  For bf16/fp16 the p of
@@ -118,17 +118,13 @@ struct DecodeShape {
   static constexpr int kL = kRowBytes / 32;    // lanes per K row
   static constexpr int kGpw = kWave / kL;      // K rows per wave load
   static constexpr int kTile = TILE >= 2 * kGpw ? TILE : 2 * kGpw;
-  static constexpr int kLog2Gpw = kGpw == 4 ? 2 : kGpw == 8 ? 3 : kGpw == 16 ? 4 : kGpw == 32 ? 5 : 6;
+  static constexpr int kLog2Gpw = kGpw == 4 ? 2 : 3;
   static constexpr int kTpg = kTile / kGpw;    // tile tokens per row group
-  // PV layout
-  static constexpr int kPvBytes = (kRowBytes / kWave) >= 4 ? (kRowBytes / kWave) : 4;
-  static constexpr int kLp = kRowBytes / kPvBytes;  // lanes per V row
-  static constexpr int kR = kWave / kLp;            // V rows per wave load
-  static constexpr int kPe = kPvBytes / kE;         // elements per lane
-  static constexpr int kRows = kTile / kR;          // V loads per lane per tile
-  static_assert(kL >= 1 && kL <= 16, "row must be 32..512 bytes");
+  // PV layout: a V row per wave load
+  static constexpr int kPvBytes = kRowBytes / kWave;
+  static constexpr int kPe = kPvBytes / kE;  // elements per lane
+  static_assert(kL == 8 || kL == 16, "rows of 256 or 512 bytes");
   static_assert(kTpg >= 2 && kTpg % 2 == 0, "token pairs need an even count per group");
-  static_assert(kGpw % kR == 0, "pair partner must sit in the same lane");
 };
 
 template <int NB>
@@ -171,17 +167,13 @@ __device__ __forceinline__ float slice_dot(const uint4 (&q)[2], const uint4 (&k)
 }
 
 // Max over the lanes of a wave that share (lane % L): every row group.
-// Every step pairs lanes of equal (lane % L) only (rotations by multiples of
-// L within a row of 16, then the row and half swaps), so the lanes of one
-// row group may hold different values (the reduce-scatter score layout).
+// Every step pairs lanes of equal (lane % L) only (a rotation by 8 within a
+// row of 16, then the row and half swaps), so the lanes of one row group may
+// hold different values (the reduce-scatter score layout).
 template <int L>
 __device__ __forceinline__ float across_groups_max(float x) {
-  if constexpr (L <= 1) x = fmaxf(x, dpp<kDppRowRor1>(x));
-  if constexpr (L <= 2) x = fmaxf(x, dpp<kDppRowRor2>(x));
-  if constexpr (L <= 4) x = fmaxf(x, dpp<kDppRowRor4>(x));
-  if constexpr (L <= 8) x = fmaxf(x, dpp<kDppRowRor8>(x));
-  if constexpr (L <= 16) x = max_row_pairs(x);
-  return max_halves(x);
+  if constexpr (L == 8) x = fmaxf(x, dpp<kDppRowRor8>(x));
+  return max_halves(max_row_pairs(x));
 }
 
 // SHARED: the workgroup is one of several sub-groups of a KV head's query
@@ -208,24 +200,19 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
   constexpr int TPG = S::kTpg;
   constexpr int CE = S::kChunkElems;
   constexpr int PE = S::kPe;
-  constexpr int R = S::kR;
-  constexpr int ROWS = S::kRows;
   constexpr bool HALF = S::kHalf;  // 16-bit elements (bf16 or fp16)
   // p staging per wave: 16-bit pairs [16 pairs][G] or fp32 [32 tokens][G]
   constexpr int kTile = S::kTile;
   constexpr int PWORDS = HALF ? (kTile / 2) * G : kTile * G;
   constexpr bool MASKD = DM < D;
   constexpr int KPM = DM / S::kChunkElems;  // 16-byte pieces of a row in memory
-  static_assert(!MASKD || (DM % S::kChunkElems == 0 && KPM >= S::kL && DM % S::kPe == 0),
-                "masked head dims: whole 16-byte pieces, at least one piece per lane");
-  // RS: reduce-scatter scores, for groups of more than half a row
-  // group of lanes (L of 4 or 8): NP score positions (G rounded up to a power
-  // of two, at least L), and lane lig of every row group ends with the
-  // scores of its HPL query heads lig*HPL .. lig*HPL + HPL-1 alone (see
-  // qk_softmax_rs).
-  constexpr bool RS = (L == 4 || L == 8) && G > L / 2;
-  constexpr int NP = !RS ? 1 : (G <= L ? L : 8);
-  constexpr int HPL = RS ? NP / L : 1;
+  static_assert(!MASKD || (!HALF && DM % S::kChunkElems == 0 && KPM >= S::kL && DM % S::kPe == 0),
+                "masked head dims: fp32, whole 16-byte pieces, at least one piece per lane");
+  // RS: reduce-scatter scores, for groups of more than half a row group of 8
+  // lanes: a score position per lane, and lane lig of every row group ends
+  // with the scores of query head lig alone (see qk_softmax_rs).
+  constexpr bool RS = L == 8 && G > 4;
+  static_assert(!RS || (!HALF && G <= 8), "rows of 256 bytes are fp32 heads of 64");
 
   // Block ids of the partition; its tail from kParkStart holds the new
   // token's pieces and their destinations from the staging to the last tile
@@ -233,7 +220,7 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
   constexpr int kBlkInts = kMaxPartition + 2;
   constexpr int kParkStart = (kBlkInts - kWave * 6) & ~3;  // 16-byte aligned
   __shared__ __align__(16) int s_blk[kBlkInts];
-  __shared__ uint4 s_q[(RS ? NP : G) * D * S::kE / 16];
+  __shared__ uint4 s_q[(RS ? L : G) * D * S::kE / 16];
   __shared__ uint32_t s_p[kDecodeWaves][PWORDS];
   __shared__ float s_m[kDecodeWaves][G];
   __shared__ float s_l[kDecodeWaves][G];
@@ -333,12 +320,10 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
     const int b = row_ok && col < a.block_table_stride ? a.block_tables[trow * a.block_table_stride + col] : -1;
     if (b >= 0 && b < a.total_blocks) {
       const bool is_v = lane >= kAppendPieces;
-      const int g = append_elem(lane);  // element in the token's row
-      const int h = g / a.head_dim;
       const T* src = reinterpret_cast<const T*>(is_v ? a.new_value : a.new_key) +
                      qtok * (is_v ? a.new_value_token_stride : a.new_key_token_stride) +
-                     static_cast<int64_t>(h) * (is_v ? a.new_value_head_stride : a.new_key_head_stride) +
-                     (g - h * a.head_dim);
+                     static_cast<int64_t>(kvh) * (is_v ? a.new_value_head_stride : a.new_key_head_stride) +
+                     (append_elem(lane) - kvh * DM);
       append_dst = append_target(b, lane);
       append_piece = ld16(src);
     }
@@ -349,16 +334,15 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
   const int lig = lane % L;  // lane within its row group
   const int gi = lane / L;   // row group within the wave
   constexpr int QCHUNKS = G * D / CE;  // 16-byte pieces of the G query rows
-  constexpr int QN = RS ? 2 * L * NP : QCHUNKS;  // 16-byte pieces staged
+  constexpr int QN = RS ? 2 * L * L : QCHUNKS;  // 16-byte pieces staged
   auto query_piece = [&](int i) -> uint4 {
     if constexpr (RS) {
       // Per (position p, lane l) of a row group, the two pieces (l and l + L)
-      // lane l dots at position p: those of query head p ^ (l * HPL), zero
-      // past G.  A lane's reads for p = 0 .. NP-1 are then one base address
-      // plus constants.
+      // lane l dots at position p: those of query head p ^ l, zero past G.  A
+      // lane's reads for p = 0 .. 7 are then one base address plus constants.
       const int piece = i & 1;
       const int ln = (i >> 1) % L;
-      const int g = ((i >> 1) / L) ^ (ln * HPL);
+      const int g = ((i >> 1) / L) ^ ln;
       const T* qrow = reinterpret_cast<const T*>(a.query) + qtok * a.q_token_stride +
                       static_cast<int64_t>(h0 + min(g, G - 1)) * a.q_head_stride;
       return (g < G && (!MASKD || ln + piece * L < KPM)) ? ld16(qrow + (ln + piece * L) * CE)
@@ -402,8 +386,6 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
   __syncthreads();
 
   const float scale = a.scale_log2e;
-  const int sub = lane / S::kLp;  // V row of this lane within a wave load
-  const int lp = lane % S::kLp;   // head-dimension slice of this lane
   float m[G], acc[G][PE];
 #pragma unroll
   for (int g = 0; g < G; ++g) m[g] = kScoreFloor;
@@ -423,13 +405,11 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
   float lsum[G];  // this lane's share of the softmax denominators
 #pragma unroll
   for (int j = 0; j < G; ++j) lsum[j] = 0.f;
-  float ml[HPL];  // RS: running maxima of the lane's own heads (sums in lsum[0 .. HPL-1])
-#pragma unroll
-  for (int h = 0; h < HPL; ++h) ml[h] = kScoreFloor;
+  float ml = kScoreFloor;  // RS: running maximum of the lane's own head (its sum in lsum[0])
 
   uint4 kb[TPG][2];
   bool kok[TPG];
-  VR vb[ROWS];
+  VR vb[kTile];
 
   auto tile_blocks = [&](int tile) {
     const int t = tile * kTile + (lane & (kTile - 1));
@@ -478,28 +458,28 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
       }
     }
   };
-  // V rows.  Fast path (one V row per wave load, blocks of >= 16 tokens):
+  // V rows.  Fast path (blocks of >= 16 tokens):
   // rows come in runs of 16 consecutive tokens inside one block, so the
   // block lookup and the 64-bit row address are formed once per run in
   // scalar registers and each further row is one scalar pointer increment.
   // Rows past the end of the partition are zeroed (p = 0 must not meet
   // uninitialised cache contents).
   constexpr int kRun = 16;
-  const bool v_runs = R == 1 && log2_bs >= 4;
+  const bool v_runs = log2_bs >= 4;
   // Element offset of the lane's V slice (formed at each use: a value kept
   // across the loop costs registers).
   auto v_slice = [&]() -> int {
     if constexpr (MASKD) {
-      return lp * PE < DM ? lp * PE : 0;
+      return lane * PE < DM ? lane * PE : 0;
     } else {
-      return lp * PE;
+      return lane * PE;
     }
   };
   auto issue_v = [&](int tile, int blk_lane, bool full) {
     const int t0 = tile * kTile;
     if (v_runs) {
 #pragma unroll
-      for (int run = 0; run < ROWS / kRun; ++run) {
+      for (int run = 0; run < kTile / kRun; ++run) {
         const int b = __builtin_amdgcn_readlane(blk_lane, run * kRun);
         if (b >= 0) {
           const int64_t slot0 =
@@ -526,18 +506,10 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
       }
     } else {
 #pragma unroll
-      for (int u = 0; u < ROWS; ++u) {
-        int b;
-        int t;
-        if constexpr (R == 1) {
-          t = t0 + u;
-          b = __builtin_amdgcn_readlane(blk_lane, u);
-        } else {
-          t = t0 + R * u + sub;
-          b = __shfl(blk_lane, R * u + sub, kWave);
-        }
+      for (int u = 0; u < kTile; ++u) {
+        const int b = __builtin_amdgcn_readlane(blk_lane, u);
         if (b >= 0) {
-          const int64_t slot = (static_cast<int64_t>(b) << log2_bs) | ((p0 + t) & bs_mask);
+          const int64_t slot = (static_cast<int64_t>(b) << log2_bs) | ((p0 + t0 + u) & bs_mask);
           vb[u] = kv_load<VR, kNt>(vbase + slot * row_stride + v_slice());
         } else {
           vb[u] = VR{};
@@ -550,70 +522,50 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
   // Scores stay unscaled (the max commutes with the positive scale); the
   // scale is applied inside the exponent: p = exp2(s * scale - max * scale).
   //
-  // RS layout: position p of lane lig dots the query head p ^ (lig * HPL),
-  // so after the NP partial dots every lane holds one partial of each head.
-  // Halving steps over the row group each add the partner lane's partial of
-  // the heads the lane keeps: partners lig ^ 7 (row half-mirror), ^ 2, ^ 1
-  // for rows of 8 lanes; lig ^ 2, ^ 1 for rows of 4.  The partner holds head
-  // h at position h ^ ((lig ^ c) * HPL), so for a kept position p it is
-  // p ^ (c * HPL), in the discarded half.  After the steps (NP - HPL adds
-  // instead of log2(L) per head) positions 0 .. HPL-1 of lane lig hold the
-  // scores of heads lig*HPL + h.  The tile maxima are then HPL reductions
-  // over the row groups, and the lane computes, sums and stages its own
-  // heads' exponentials with no selection among heads.
+  // RS layout: position p of lane lig dots the query head p ^ lig, so after
+  // the 8 partial dots every lane holds one partial of each head.  Halving
+  // steps over the row group each add the partner lane's partial of the heads
+  // the lane keeps: partners lig ^ 7 (row half-mirror), ^ 2, ^ 1.  The partner
+  // holds head h at position h ^ (lig ^ c), so for a kept position p it is
+  // p ^ c, in the discarded half.  After the steps (7 adds instead of 3 per
+  // head) position 0 of lane lig holds the score of head lig.  The tile maxima
+  // are then one reduction over the row groups, and the lane computes, sums
+  // and stages its own head's exponentials with no selection among heads.
   auto qk_softmax_rs = [&](bool full) {
-    float s[TPG][HPL];
+    float s[TPG];
     {
-      float x[TPG][NP];
+      float x[TPG][L];
       const uint4* sq = s_q + 2 * lig;
 #pragma unroll
-      for (int p = 0; p < NP; ++p) {
+      for (int p = 0; p < L; ++p) {
         const uint4 qg[2] = {sq[2 * L * p], sq[2 * L * p + 1]};
 #pragma unroll
         for (int i = 0; i < TPG; ++i) x[i][p] = slice_dot<T>(qg, kb[i]);
       }
 #pragma unroll
       for (int i = 0; i < TPG; ++i) {
-        if constexpr (L == 8) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) x[i][q] += dpp<kDppRowHalfMirror>(x[i][q ^ 7]);
+        for (int q = 0; q < 4; ++q) x[i][q] += dpp<kDppRowHalfMirror>(x[i][q ^ 7]);
 #pragma unroll
-          for (int q = 0; q < 2; ++q) x[i][q] += dpp<kDppQuadXor2>(x[i][q ^ 2]);
-          x[i][0] += dpp<kDppQuadXor1>(x[i][1]);
-        } else if constexpr (NP == 4) {
-#pragma unroll
-          for (int q = 0; q < 2; ++q) x[i][q] += dpp<kDppQuadXor2>(x[i][q ^ 2]);
-          x[i][0] += dpp<kDppQuadXor1>(x[i][1]);
-        } else {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) x[i][q] += dpp<kDppQuadXor2>(x[i][q ^ 4]);
-#pragma unroll
-          for (int q = 0; q < 2; ++q) x[i][q] += dpp<kDppQuadXor1>(x[i][q ^ 2]);
-        }
-#pragma unroll
-        for (int h = 0; h < HPL; ++h) s[i][h] = (full || kok[i]) ? x[i][h] : -INFINITY;
+        for (int q = 0; q < 2; ++q) x[i][q] += dpp<kDppQuadXor2>(x[i][q ^ 2]);
+        x[i][0] += dpp<kDppQuadXor1>(x[i][1]);
+        s[i] = (full || kok[i]) ? x[i][0] : -INFINITY;
       }
     }
-    // Head lig*HPL + h's tile maximum, in every row group; head g's is read
-    // from lane g / HPL (row group 0).
-    float tm[HPL];
+    // Head lig's tile maximum, in every row group; head g's is read from lane
+    // g (row group 0).
+    float tm = s[0];
 #pragma unroll
-    for (int h = 0; h < HPL; ++h) {
-      tm[h] = s[0][h];
-#pragma unroll
-      for (int i = 1; i < TPG; ++i) tm[h] = fmaxf(tm[h], s[i][h]);
-      tm[h] = across_groups_max<L>(tm[h]);
-    }
+    for (int i = 1; i < TPG; ++i) tm = fmaxf(tm, s[i]);
+    tm = across_groups_max<L>(tm);
     bool moved = false;
     float m_new[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      m_new[g] = fmaxf(m[g], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tm[g % HPL]), g / HPL)));
+      m_new[g] = fmaxf(m[g], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tm), g)));
       moved |= m_new[g] != m[g];
     }
-    float ml_new[HPL];  // m_new of the lane's heads (those below G)
-#pragma unroll
-    for (int h = 0; h < HPL; ++h) ml_new[h] = fmaxf(ml[h], tm[h]);
+    const float ml_new = fmaxf(ml, tm);  // m_new of the lane's head (those below G)
     if (moved) {  // wave-uniform
       float alpha[G];
 #pragma unroll
@@ -621,36 +573,21 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
         alpha[g] = fast_exp2((m[g] - m_new[g]) * scale);
         m[g] = m_new[g];
       }
-#pragma unroll
-      for (int h = 0; h < HPL; ++h) lsum[h] *= fast_exp2((ml[h] - ml_new[h]) * scale);
+      lsum[0] *= fast_exp2((ml - ml_new) * scale);
 #pragma unroll
       for (int j = 0; j < G; ++j)
 #pragma unroll
         for (int e = 0; e < PE; ++e) acc[j][e] *= alpha[j];
     }
     uint32_t* sp = s_p[wave];
+    ml = ml_new;
+    const float mc = -ml * scale;
+    if (lig < G) {
 #pragma unroll
-    for (int h = 0; h < HPL; ++h) {
-      ml[h] = ml_new[h];
-      const float mc = -ml[h] * scale;
-      const int head = lig * HPL + h;
-      if (head < G) {
-        if constexpr (HALF) {
-#pragma unroll
-          for (int k = 0; k < TPG / 2; ++k) {
-            const float pa = fast_exp2(fmaf(s[2 * k][h], scale, mc));
-            const float pb = fast_exp2(fmaf(s[2 * k + 1][h], scale, mc));
-            lsum[h] += pa + pb;
-            sp[(k * GPW + gi) * G + head] = pack_half2<T>(pa, pb);
-          }
-        } else {
-#pragma unroll
-          for (int i = 0; i < TPG; ++i) {
-            const float pa = fast_exp2(fmaf(s[i][h], scale, mc));
-            lsum[h] += pa;
-            sp[(gi + GPW * i) * G + head] = __float_as_uint(pa);
-          }
-        }
+      for (int i = 0; i < TPG; ++i) {
+        const float pa = fast_exp2(fmaf(s[i], scale, mc));
+        lsum[0] += pa;
+        sp[(gi + GPW * i) * G + lig] = __float_as_uint(pa);
       }
     }
     __builtin_amdgcn_wave_barrier();
@@ -736,11 +673,9 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
   auto pv = [&]() {
     const uint32_t* sp = s_p[wave];
     if constexpr (HALF) {
-      constexpr int PARTNER = GPW / R;  // V load holding token t + GPW
 #pragma unroll
-      for (int u = 0; u < ROWS; ++u) {
-        if (((R * u) % (2 * GPW)) >= GPW) continue;
-        const int t = R * u + sub;
+      for (int t = 0; t < kTile; ++t) {
+        if (t % (2 * GPW) >= GPW) continue;
         const int pidx = (t / (2 * GPW)) * GPW + (t % GPW);
         uint32_t pw[G];
 #pragma unroll
@@ -748,7 +683,7 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
 #pragma unroll
         for (int w = 0; w < PE / 2; ++w) {
           // Element 2w (lo) and 2w+1 (hi) of tokens t and t + GPW, paired.
-          const uint32_t va = v_word(vb[u], w), vbb = v_word(vb[u + PARTNER], w);
+          const uint32_t va = v_word(vb[t], w), vbb = v_word(vb[t + GPW], w);
           const uint32_t lo = __builtin_amdgcn_perm(vbb, va, 0x05040100u);
           const uint32_t hi = __builtin_amdgcn_perm(vbb, va, 0x07060302u);
 #pragma unroll
@@ -760,14 +695,13 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
       }
     } else {
 #pragma unroll
-      for (int u = 0; u < ROWS; ++u) {
-        const int t = R * u + sub;
+      for (int t = 0; t < kTile; ++t) {
         float v[PE];
         if constexpr (PE == 1) {
-          v[0] = __uint_as_float(vb[u]);
+          v[0] = __uint_as_float(vb[t]);
         } else {
-          v[0] = __uint_as_float(vb[u].x);
-          v[1] = __uint_as_float(vb[u].y);
+          v[0] = __uint_as_float(vb[t].x);
+          v[1] = __uint_as_float(vb[t].y);
         }
 #pragma unroll
         for (int g = 0; g < G; ++g) {
@@ -821,24 +755,15 @@ __global__ __launch_bounds__(kDecodeThreads) PA_DECODE_OCCUPANCY(T, D, G) void d
   float ltot[G];
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    float l = RS ? (lig == g / HPL ? lsum[g % HPL] : 0.f) : lsum[g];
+    float l = RS ? (lig == g ? lsum[0] : 0.f) : lsum[g];
 #pragma unroll
     for (int o = kWave / 2; o >= 1; o >>= 1) l += __shfl_xor(l, o, kWave);
     ltot[g] = l;
   }
-  // V rows of one wave load that hold different tokens -> add them up.
 #pragma unroll
-  for (int o = kWave / 2; o >= S::kLp; o >>= 1)
+  for (int j = 0; j < G; ++j)
 #pragma unroll
-    for (int j = 0; j < G; ++j)
-#pragma unroll
-      for (int e = 0; e < PE; ++e) acc[j][e] += __shfl_xor(acc[j][e], o, kWave);
-  if (sub == 0) {
-#pragma unroll
-    for (int j = 0; j < G; ++j)
-#pragma unroll
-      for (int e = 0; e < PE; ++e) s_acc[wave][j * D + lp * PE + e] = acc[j][e];
-  }
+    for (int e = 0; e < PE; ++e) s_acc[wave][j * D + lane * PE + e] = acc[j][e];
   if (lane < G) {
 #pragma unroll
     for (int g = 0; g < G; ++g)

@@ -49,7 +49,6 @@ struct DecodeArgs {
   int64_t new_key_head_stride;
   int64_t new_value_token_stride;
   int64_t new_value_head_stride;
-  int32_t head_dim;
   // Merge records of the in-launch split-K merge, 8 bytes per (sequence,
   // unit, sub-group): arrivals, first full-partition item, partial item.
   // Zero before the launch and left zero by it; null (always for 65535 or
