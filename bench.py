@@ -56,7 +56,7 @@ inside the decode launch) from eager launches and from one HIP graph of the
 
 --workload decode_partitions prints, for latency-bound decode steps in a
 32-layer loop, the per-layer time of every split-K partition from 64 to 4096
-and the partition pa_plan_step picks.
+and the partition pack_step picks.
 
 --ab-library PATH [--ab-rounds N] times the workload's kernels and step in
 alternation with another build of the library (csrc/build.py --rev REV
@@ -365,6 +365,14 @@ def measured_traffic(workload: str):
     return int(entry["traffic_bytes"]) if entry else None
 
 
+def decode_kernel(w) -> str:
+    """The kernel the decode of a workload launches (its partition phase)."""
+    import torch
+
+    on_matrix_cores = w.dtype != torch.float32 and w.head_dim in (64, 80, 96, 128)
+    return "decode_mfma_kernel" if on_matrix_cores else "decode_partition_kernel"
+
+
 def workload_config(w, **extra):
     cfg = {
         "workload": w.name,
@@ -606,7 +614,7 @@ def decode_main(args, w, t, device):
                                      "HIP graph, medians"},
         "roofline": {
             "bound": "hbm",
-            "kernel": "decode_partition_kernel",
+            "kernel": decode_kernel(w),
             "achieved": round(kernel_gbs, 2),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
@@ -761,7 +769,7 @@ def decode_config_line(args, w, t, device):
         "value": round(gbs, 2), "unit": "GB/s", "hbm_frac": round(gbs / HBM_PEAK_GBS, 4),
         "ms_per_step": round(ms, 5), "tokens_per_s": round(w.num_query_tokens / (ms * 1e-3), 1), "dtype": "bf16",
         "partition": step.partition_size, "config": workload_config(w),
-        "roofline": {"bound": "hbm", "kernel": "decode_partition_kernel",
+        "roofline": {"bound": "hbm", "kernel": decode_kernel(w),
                      "achieved": round(kernel_gbs, 2), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(kernel_gbs / HBM_PEAK_GBS, 4),
                      "traffic": measured_traffic(w.name),
@@ -852,7 +860,7 @@ def mixed_line(args, w, t, device):
                    "attention_ms": round(att1, 5), "with_kv_write_ms": round(wr1, 5), "full_step_ms": round(full2, 5)},
         "full_step_tokens_per_s": round(w.num_query_tokens / (full_ms * 1e-3), 1), "dtype": "bf16",
         "partition": step.partition_size, "config": workload_config(w),
-        "decode": {"kernel": "decode_partition_kernel", "kernel_ms": round(decode_kernel_ms, 5),
+        "decode": {"kernel": decode_kernel(w), "kernel_ms": round(decode_kernel_ms, 5),
                    "gbs": round(kv_bytes / (decode_kernel_ms * 1e-3) / 1e9, 2),
                    "hbm_frac": round(kv_bytes / (decode_kernel_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                    "traffic": measured_traffic(w.name), "algorithmic_bytes": kv_bytes,
@@ -1006,7 +1014,7 @@ def decode_partitions_line(args, device):
     cache read cold, each layer writing its new rows inside the decode
     launch): per-layer time of each split-K partition from 64 to 4096 from
     one HIP graph of 10 passes, 7 alternated rounds, medians; beside it the
-    partition pa_plan_step picks and how far it is from the fastest."""
+    partition pack_step picks and how far it is from the fastest."""
     import numpy as np
     import torch
 

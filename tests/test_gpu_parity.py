@@ -424,8 +424,9 @@ def test_decode_occupancy_query(device):
 
 
 def test_pack_step_partition_uses_the_kernel_queries(device):
-    """pack_step's automatic partition is choose_partition fed with the
-    library's launch-shape queries and the device's compute units."""
+    """On a step that fills the chip, pack_step's automatic partition is
+    choose_partition fed with the library's launch-shape queries and the
+    device's compute units, in every dtype."""
     for hq, hkv, d, dtype in ((32, 8, 128, torch.bfloat16), (8, 8, 128, torch.float32),
                               (128, 8, 128, torch.bfloat16), (16, 8, 64, torch.float16)):
         w = wl.llama3_8b_gqa_decode(seed=0)

@@ -574,3 +574,16 @@ def test_which_steps_write_prefill_rows_in_the_prefill_launch(dtype, starts, cou
                          num_query_tokens=sum(counts), num_seqs=len(counts), max_new_tokens=max(counts),
                          num_decode_items=sum(c == 1 for c in counts), num_prefill_items=sum(c > 1 for c in counts))
     assert ops._writes_in_prefill(torch.empty(0, dtype=dtype), step) is inside
+
+
+@pytest.mark.parametrize("workload", ["llama3_8b_gqa_decode", "llama7b_mha_decode", "mixed_step"])
+def test_bench_names_the_kernel_whose_traffic_it_quotes(workload):
+    import json
+    from pathlib import Path
+
+    import bench
+
+    w = pkg("workloads").WORKLOADS[workload](seed=0)
+    table = json.loads((Path(bench.__file__).parent / "profiles" / "pmc_traffic.json").read_text())
+    assert "::" + bench.decode_kernel(w) + "<" in table[workload]["kernel"]
+    assert bench.measured_traffic(workload) == table[workload]["traffic_bytes"] >= table[workload]["algorithmic_bytes"]
