@@ -91,7 +91,7 @@ int64_t choose_partition(const DecodeContexts& d, const PaPlanParams& p, int64_t
 // Constants per head dim, fitted to 928 steps of 1-160 sequences of 4-65536
 // tokens, 27 head shapes, from a HIP graph over cold layers, where the picks take
 // 1.2 % longer than the best power of two on average and 20 % at most (the model
-// above: 13 % and 104 %).  Two failures of a model of one constant rate a
+// above: 12 % and 91 %).  Two failures of a model of one constant rate a
 // workgroup and no share of the last ones: 49 sequences of 748-1648 tokens, 8/8
 // heads of 64, at 2048, 30.4 us (26.7 at 256); 21 of 7331-15987, 8/8 heads of 128,
 // at 4096, 175 us (165 at 1024).
@@ -105,7 +105,7 @@ struct MfmaModel {
 constexpr double kHbmBytesPerUs = 6.7e6;
 constexpr int64_t kMfmaRoundTokens = 128;
 constexpr int64_t kMinFullChipMfmaPartition = 1024;
-constexpr MfmaModel kMfmaModel128 = {1.45, 0.02, 0.00027, 1.9, 1.4};
+constexpr MfmaModel kMfmaModel128 = {1.45, 0.012, 0.00025, 2.3, 1.4};
 constexpr MfmaModel kMfmaModel64 = {1.19, 0.26, 0.0007, 0.63, 2.0};
 // Heads of 80 and 96, whose rows share cache lines with the next head's: two
 // sequences of 20142-27521 tokens, 32/8 heads of 96, 35.2 us at its 2048 (40.4
