@@ -264,10 +264,11 @@ int pa_plan_step(const int64_t *start_positions, const int64_t *new_token_counts
 /*
  * pa_plan_step for a cache dtype and head dim: where partition_size is 0 and
  * the shape's decode runs on the matrix cores (16-bit heads of 64, 80, 96 and
- * 128), a launch that does not fill the chip at 2048 tokens or more takes the
+ * 128), a launch that does not fill the chip at 1024 tokens or more takes the
  * partition of 64 ... 4096 (a power of two) of least modelled time for that
  * kernel, from the step's bytes, its workgroups, the largest of them and the
- * longest sequence's partials; heads of 80 and 96 have constants of their own.
+ * longest sequence's partials, with constants for heads of 64, of 80 and 96 and
+ * of 128.
  * Any other dtype or head dim: pa_plan_step.
  */
 int pa_plan_step_for(const int64_t *start_positions, const int64_t *new_token_counts,
@@ -358,14 +359,18 @@ size_t pa_decode_workspace_size(PaStepDims dims, int64_t num_decode_items);
  * counterpart in the reference.) */
 size_t pa_decode_merge_state_size(PaStepDims dims, int64_t num_decode_items);
 
-/* Partition workgroups pa_decode launches per decode work item:
+/* Partition workgroups of pa_decode per decode work item:
  *  - num_kv_heads / 2 when two adjacent KV heads run as one workgroup
  *    (bf16 or fp16, an even KV head count, head_dim 64 or 128 and groups of up to 4
  *    query heads: each token's rows of the two heads are read as one row of
  *    twice the length);
  *  - num_kv_heads x the sub-groups of a group of more than 8 query heads
- *    (the fewest equal sub-groups of at most 8; each reads the K/V again,
- *    ordered so that the re-reads of one KV head's rows meet one L2);
+ *    (the fewest equal sub-groups of at most 8).  fp32 heads and 16-bit heads
+ *    of 256 launch one workgroup for each, which reads the K/V again, ordered
+ *    so that the re-reads of one KV head's rows meet one L2; the matrix cores
+ *    (16-bit heads of 64, 80, 96 and 128) take up to 16 query heads in one
+ *    workgroup, which counts as its sub-groups, as pa_decode_workgroups_per_cu
+ *    counts it too;
  *  - num_kv_heads otherwise; 0 for head counts pa_decode rejects.
  * A host choosing the split-K partition size from the launch width uses it.
  * (No counterpart in the reference, whose CPU kernel has no workgroups.) */

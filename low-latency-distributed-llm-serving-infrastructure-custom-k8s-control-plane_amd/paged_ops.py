@@ -417,9 +417,12 @@ _DECODE_CUS = 256
 
 def decode_workgroups_per_item(dtype: torch.dtype, head_dim: int, num_kv_heads: int,
                                num_query_heads: int) -> int:
-    """Partition workgroups the decode launches per work item: half the KV
-    heads when adjacent heads run as pairs, KV heads x sub-groups for groups
-    of more than 8 query heads, else the KV heads (0 for rejected counts)."""
+    """Partition workgroups of the decode per work item: half the KV heads
+    when adjacent heads run as pairs, KV heads x sub-groups of at most 8 for
+    groups of more than 8 query heads, else the KV heads (0 for rejected
+    counts).  16-bit heads of 64, 80, 96 and 128 run two sub-groups in one
+    workgroup, which counts as two here and in
+    :func:`decode_workgroups_per_cu`."""
     return _workgroups_per_item(dtype_code(dtype), int(head_dim), int(num_kv_heads), int(num_query_heads))
 
 
@@ -497,6 +500,11 @@ def choose_partition(
     16384 tokens, bf16 and fp32, groups of 4 and 8) the pick is the fastest
     partition on 17 and within 9.2 % on the rest; e.g. two sequences of 8192
     tokens 26.7 us per layer at 256 (the earlier rule's 128: 29.7).
+
+    These read rates are the vector kernel's.  :func:`pack_step` knows the
+    cache dtype and head dim and asks ``pa_plan_step_for``, which has a model
+    of the matrix-core decode (16-bit heads of 64, 80, 96 and 128) for steps
+    that do not fill the chip at 1024 tokens or more; its pick can differ there.
     """
     p = _plan(_int64_array(start_positions), _int64_array(new_token_counts), 1, 1, 0, num_kv_heads,
               num_query_heads or 0, workgroups_per_item or 0, workgroups_per_cu or 0, compute_units)
